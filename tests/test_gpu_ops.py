@@ -33,6 +33,92 @@ def test_gemm_f32(ctx, orc, M, N, K, ta, tb):
         assert rel_err(got, ref) <= 1e-3, (alpha, beta)
 
 
+def _gemm64(A, B):
+    """(A.B, |A|.|B|) in 64 bits: f32 sums of K products in any order differ from
+    the first by at most (K + slices + 2) eps of the second."""
+    return A.astype(np.float64) @ B.astype(np.float64), np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)
+
+
+@pytest.mark.parametrize("M,N,K,pad,off", [
+    (32, 128, 64, 0, 0), (33, 129, 65, 0, 0), (31, 127, 63, 0, 0), (1, 1, 1, 0, 0),      # tile edges
+    (64, 64, 128, 4, 0), (65, 63, 132, 4, 0), (4, 260, 4096, 8, 0),                       # padded rows, 16-byte loads
+    (40, 72, 260, 3, 0), (40, 72, 260, 4, 1), (2, 130, 1000, 0, 3),                       # odd rows, odd addresses
+    (100, 200, 6000, 0, 0), (1, 100, 8191, 0, 0), (700, 768, 1000, 0, 0),                 # split K, ragged slices
+])
+@pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False), (True, True)])
+def test_gemm_f32_tiles_and_splits(ctx, M, N, K, pad, off, ta, tb):
+    """Edges of the tiles, of the K steps and of the slices; leading dimensions
+    beyond the rows; addresses that forbid 16-byte loads."""
+    print(f"[case] gemm_f32 {M}x{N}x{K} pad={pad} off={off} ta={ta} tb={tb}", flush=True)
+    A, B = (F.normal(64, n, r * c).reshape(r, c) for n, r, c in ((f"a{M}.{K}", M, K), (f"b{K}.{N}", K, N)))
+
+    def put(X, trans):
+        X = X.T if trans else X
+        rows, cols = X.shape
+        host = np.full(off + rows * (cols + pad), np.nan, np.float32)   # the padding is not used
+        host[off:].reshape(rows, cols + pad)[:, :cols] = X
+        return ctx.to_device(host), cols + pad
+
+    (dA, lda), (dB, ldb) = put(A, ta), put(B, tb)
+    ldc = N + pad
+    C0 = F.normal(64, f"c{M}.{N}", M * ldc).reshape(M, ldc)
+    dC = ctx.to_device(C0)
+    V.check(V.lib().vlrf_hip_gemm_f32(ctx.h, dA.ptr + 4 * off, dB.ptr + 4 * off, dC.ptr, M, N, K, lda, ldb, ldc,
+                                      1.5, 0.5, int(ta), int(tb)))
+    got = dC.download((M, ldc))
+    ref, mag = _gemm64(A, B)
+    bound = (K + 70) * 2.0 ** -24 * 1.5 * mag + 3 * 2.0 ** -24 * np.abs(0.5 * C0[:, :N].astype(np.float64)) + 1e-30
+    assert (np.abs(got[:, :N] - (1.5 * ref + 0.5 * C0[:, :N])) <= bound).all()
+    assert np.array_equal(got[:, N:], C0[:, N:])                        # between the rows of C
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 40, 200), (70, 130, 1024)])
+def test_gemm_f32_specials(ctx, M, N, K):
+    """Infinities, NaN and denormals stay in their row of C and keep their meaning."""
+    A, B = F.normal(65, f"sa{K}", M * K).reshape(M, K), F.normal(65, f"sb{K}", N * K).reshape(N, K)
+    A[0, 1], A[1, K - 1], A[2] = np.inf, np.nan, 0.0
+    A[2, 0], B[0] = 1e-39, 0.0                                          # a denormal times 2 is exact in f32
+    B[0, 0] = 2.0
+    dA, dB, dC = ctx.to_device(A), ctx.to_device(B), ctx.alloc(M * N * 4)
+    ctx.gemm_f32(dA, dB, dC, M, N, K, trans_b=True)
+    got = dC.download((M, N))
+    ref, mag = _gemm64(A[2:], B.T)
+    assert (np.isinf(got[0, 1:]).all() and (np.sign(got[0, 1:]) == np.sign(B[1:, 1])).all())
+    assert np.isnan(got[0, 0]) and np.isnan(got[1]).all()               # inf * 0, NaN
+    assert (np.abs(got[2:] - ref) <= (K + 70) * 2.0 ** -24 * mag + 1e-45).all()
+    assert got[2, 0] == np.float32(1e-39) * np.float32(2.0)
+
+
+def test_gemm_f32_under_graph_capture():
+    """Under capture K stays whole (a captured launch keeps no scratch address
+    that a later call may regrow); every replay gives the same result."""
+    import ctypes as C
+    from test_gpu_prefill_gemm import _hip
+    hip, ctx = _hip(), V.Context(0)
+    M, N, K = 60, 100, 4096
+    A, B = F.normal(66, "ca", M * K).reshape(M, K), F.normal(66, "cb", N * K).reshape(N, K)
+    dA, dB, dC, dE = ctx.to_device(A), ctx.to_device(B), ctx.alloc(M * N * 4), ctx.alloc(M * N * 4)
+    ctx.gemm_f32(dA, dB, dE, M, N, K, trans_b=True)
+    eager = dE.download((M, N))
+    s, g, ge = C.c_void_p(ctx.stream()), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(s, 2) == 0
+    rc = V.lib().vlrf_hip_gemm_f32(ctx.h, dA.ptr, dB.ptr, dC.ptr, M, N, K, K, K, N, 1.0, 0.0, 0, 1)
+    assert hip.hipStreamEndCapture(s, C.byref(g)) == 0 and rc == 0
+    assert hip.hipGraphInstantiate(C.byref(ge), g, None, None, 0) == 0
+    ref, mag = _gemm64(A, B.T)
+    big = ctx.alloc(4 * 64 * 8192)
+    for _ in range(3):
+        dC.zero()
+        ctx.gemm_f32(dA, dB, big, M, 100, K, trans_b=True)              # eager work, with scratch, between
+        assert hip.hipGraphLaunch(ge, s) == 0
+        ctx.sync()
+        got = dC.download((M, N))
+        assert (np.abs(got - ref) <= (K + 70) * 2.0 ** -24 * mag).all()
+        assert (np.abs(eager - ref) <= (K + 70) * 2.0 ** -24 * mag).all()
+    hip.hipGraphExecDestroy(ge)
+    hip.hipGraphDestroy(g)
+
+
 def test_gemm_f32_rejects_bad_shapes(ctx):
     a = ctx.alloc(64)
     with pytest.raises(V.HipError):

@@ -173,6 +173,23 @@ int vlrf_hip_ctx::scratch(size_t bytes, float** out) {
     return VLRF_HIP_OK;
 }
 
+float* vlrf_hip_ctx::try_scratch(size_t bytes) {
+    float* p = nullptr;
+    if (!bytes) return nullptr;
+    // Not under capture: a captured launch would keep the address of a buffer
+    // that a later call may regrow.
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (scratch(bytes, &p) != VLRF_HIP_OK) {
+        (void)hipGetLastError();   // the caller goes on: no error is left for its launch check
+        return nullptr;
+    }
+    return p;
+}
+
 vlrf_hip_ctx::~vlrf_hip_ctx() {
     (void)hipSetDevice(device);
     (void)hipStreamSynchronize(stream);
@@ -649,7 +666,8 @@ int vlrf_hip_qlinear_swiglu(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t wg, vlrf_hip_w
 int vlrf_hip_gemm_f32(vlrf_hip_ctx_t ctx, const float* A, const float* B, float* C, int M, int N, int K,
                       int lda, int ldb, int ldc, float alpha, float beta, int transA, int transB) {
     VH_CTX(ctx);
-    return launch_gemm_f32(ctx->stream, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, transA != 0, transB != 0);
+    float* part = ctx->try_scratch(gemm_f32_part_bytes(M, N, K));   // none: K stays whole
+    return launch_gemm_f32(ctx->stream, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, transA != 0, transB != 0, part);
 }
 
 int vlrf_hip_layer_norm(vlrf_hip_ctx_t ctx, const float* x, const float* w, const float* b, float* out,

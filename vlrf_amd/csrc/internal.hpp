@@ -172,7 +172,9 @@ int launch_rmsnorm(hipStream_t s, const float* x, const float* w, float* out, in
 
 // ---- the engine's remaining per-op backend calls (kernels/ops.hip) ---------------
 int launch_gemm_f32(hipStream_t s, const float* A, const float* B, float* C, int M, int N, int K, int lda,
-                    int ldb, int ldc, float alpha, float beta, bool transA, bool transB);
+                    int ldb, int ldc, float alpha, float beta, bool transA, bool transB, float* part = nullptr);
+// Device memory (part) launch_gemm_f32 splits K with; without it K stays whole.
+size_t gemm_f32_part_bytes(int M, int N, int K);
 int launch_layer_norm(hipStream_t s, const float* x, const float* w, const float* b, float* out, int rows, int D,
                       float eps);
 int launch_softmax(hipStream_t s, float* x, int rows, int D);

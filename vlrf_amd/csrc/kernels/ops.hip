@@ -17,60 +17,182 @@
 namespace vlrf_hip {
 namespace {
 
-// f32 GEMM: a 256-lane workgroup owns a 64x64 tile of C, each lane a 4x4 block
-// (rows ty + 16i, columns tx + 16j, so LDS reads of a wave are broadcast or
-// conflict-free); K in steps of 16 staged through LDS.  op(A)[m][k] and
-// op(B)[k][n] are gathered with the transposes applied on the way into LDS.
-constexpr int kGT = 64, kGK = 16;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
-                                                       float* C, int M, int N, int K, int lda, int ldb, int ldc,
-                                                       float alpha, float beta, int transA, int transB) {
-    __shared__ float As[kGK][kGT + 1];
-    __shared__ float Bs[kGK][kGT + 1];
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const int m0 = blockIdx.y * kGT, n0 = blockIdx.x * kGT;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += kGK) {
-        for (int i = tid; i < kGT * kGK; i += 256) {
-            // A tile element (m, k): lanes walk k fastest when A is row-major in k
-            const int r = transA ? i % kGT : i / kGK, c = transA ? i / kGT : i % kGK;
-            const int m = m0 + r, k = k0 + c;
-            float a = 0.f;
-            if (m < M && k < K) a = transA ? A[(size_t)k * lda + m] : A[(size_t)m * lda + k];
-            As[c][r] = a;
-            const int rb = transB ? i / kGK : i % kGT, cb = transB ? i % kGK : i / kGT;   // (n, k)
-            const int n = n0 + rb, kb = k0 + cb;
-            float b = 0.f;
-            if (n < N && kb < K) b = transB ? B[(size_t)n * ldb + kb] : B[(size_t)kb * ldb + n];
-            Bs[cb][rb] = b;
-        }
-        __syncthreads();
+// f32 GEMM on the f32 matrix instructions.  A 256-lane workgroup owns a BM x BN
+// tile of C (64x64, or 32x128 for M <= 32), each wave one 32x32 block of it in
+// v_mfma_f32_32x32x2_f32: 4096 operations in 64 cycles, so a SIMD's one wave
+// keeps its matrix core busy and two operand reads feed four instructions.  K
+// advances in steps of 64 through two LDS buffers, the next step's operands in
+// flight in registers while the current one is multiplied; a row's 64 values
+// are contiguous in LDS (rows 68 floats apart: 16-byte reads of eight rows hit
+// distinct banks), so lane half h takes k = 8s + 4h + 0..3 in one read (the
+// order of k within a step is the same for both operands, and otherwise free).
+// Products and sums are f32 FMAs as in the CPU loop; infinities and NaN pass
+// through; rows and columns outside the matrices are zeros that no stored
+// element reads.
+//
+// Bound by the matrix rate (157 TFLOP/s f32) while the tiles fill the chip,
+// else by the length of a workgroup's own K: the slices of a split K
+// (gridDim.z, partial sums to P, added in slice order by gemm_f32_reduce_kernel)
+// shorten it.  Measured against the vector-unit kernel before it (64x64 tiles, K
+// steps of 16): 300x3072x768 144 -> 20.8 us, 300x768x3072 583 -> 23.0; the rate
+// at 1024x1600x6400 is 108 TFLOP/s.  Steps of 64 with two register sets in
+// flight; loads behind bounds branches ran 240 against 205 us at 1024x6400x1600.
+constexpr int kGK = 64, kGS = kGK + 4;
+
+// A step's loads are branch-free (a guarded load would be waited for where its
+// branch ends): rows and k past the end read the last ones, and stage() zeroes
+// what lies past kend.  KC: k runs contiguously in memory, else the row index
+// does.  VEC: 16-byte loads, 32-bit offsets from the step's uniform base; the
+// run's length is a multiple of 4, the base and the leading dimension (below
+// 2^22) allow them.
+template <int ROWS, bool KC, bool VEC>
+__device__ __forceinline__ void gemm_f32_load(float4 (&st)[ROWS / 16], const float* __restrict__ X, int ld, int row0,
+                                              int rows, int k0, int kend) {
+    const float* base = KC ? X + (size_t)row0 * ld : X + (size_t)k0 * ld;
 #pragma unroll
-        for (int kk = 0; kk < kGK; ++kk) {
-            float a[4], b[4];
+    for (int i = 0; i < ROWS / 16; ++i) {
+        const int f = threadIdx.x + 256 * i;
+        const int r = KC ? f / (kGK / 4) : 4 * (f % (ROWS / 4));   // within the tile
+        const int k = KC ? 4 * (f % (kGK / 4)) : f / (ROWS / 4);
+        if constexpr (VEC) {
+            const uint32_t o = KC ? (uint32_t)(min(r, rows - 1 - row0) * ld) + min(k0 + k, kend - 4)
+                                  : (uint32_t)(min(k, kend - 1 - k0) * ld) + min(row0 + r, rows - 4);
+            st[i] = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(base) + 4u * o);
+        } else {
+            float v[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty + 16 * i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int m = m0 + ty + 16 * i, n = n0 + tx + 16 * j;
-            if (m < M && n < N) {
-                float* c = C + (size_t)m * ldc + n;
-                const float prev = beta == 0.f ? 0.f : (beta == 1.f ? *c : *c * beta);
-                *c = prev + alpha * acc[i][j];
+            for (int j = 0; j < 4; ++j) {
+                const int rj = min(row0 + (KC ? r : r + j), rows - 1), kj = min(k0 + (KC ? k + j : k), kend - 1);
+                v[j] = KC ? X[(size_t)rj * ld + kj] : X[(size_t)kj * ld + rj];
             }
+            st[i] = make_float4(v[0], v[1], v[2], v[3]);
         }
+    }
+}
+
+template <int ROWS, bool KC, bool TAIL>
+__device__ __forceinline__ void gemm_f32_stage(const float4 (&st)[ROWS / 16], float* s, int left) {
+#pragma unroll
+    for (int i = 0; i < ROWS / 16; ++i) {
+        const int f = threadIdx.x + 256 * i;
+        const int k = KC ? 4 * (f % (kGK / 4)) : f / (ROWS / 4);
+        float4 v = st[i];
+        if constexpr (TAIL) {
+            v.x = k < left ? v.x : 0.f;
+            v.y = k + (KC ? 1 : 0) < left ? v.y : 0.f;
+            v.z = k + (KC ? 2 : 0) < left ? v.z : 0.f;
+            v.w = k + (KC ? 3 : 0) < left ? v.w : 0.f;
+        }
+        if constexpr (KC) {
+            *reinterpret_cast<float4*>(s + (f / (kGK / 4)) * kGS + k) = v;
+        } else {
+            float* d = s + 4 * (f % (ROWS / 4)) * kGS + k;
+            d[0] = v.x;
+            d[kGS] = v.y;
+            d[2 * kGS] = v.z;
+            d[3 * kGS] = v.w;
+        }
+    }
+}
+
+template <int BM, int BN, bool TA, bool TB, bool VEC>
+__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                                                       float* C, float* __restrict__ P, int M, int N, int K, int lda,
+                                                       int ldb, int ldc, float alpha, float beta, int kslice) {
+    constexpr int WN = BN / 32;                                   // waves across the tile's columns
+    __shared__ __align__(16) float As[2][BM * kGS];
+    __shared__ __align__(16) float Bs[2][BN * kGS];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    const int kbeg = blockIdx.z * kslice, kend = min(K, kbeg + kslice);
+    const int ra = (w / WN) * 32 + (lane & 31), rb = (w % WN) * 32 + (lane & 31), h4 = 4 * (lane >> 5);
+    struct Regs {
+        float4 a[BM / 16], b[BN / 16];
+    } r0, r1;
+    auto load = [&](Regs& r, int k0) {
+        gemm_f32_load<BM, !TA, VEC>(r.a, A, lda, m0, M, k0, kend);
+        gemm_f32_load<BN, TB, VEC>(r.b, B, ldb, n0, N, k0, kend);
+    };
+    auto stage = [&](const Regs& r, int buf, int k0) {
+        if (kend - k0 >= kGK) {
+            gemm_f32_stage<BM, !TA, false>(r.a, As[buf], kGK);
+            gemm_f32_stage<BN, TB, false>(r.b, Bs[buf], kGK);
+        } else {
+            gemm_f32_stage<BM, !TA, true>(r.a, As[buf], kend - k0);
+            gemm_f32_stage<BN, TB, true>(r.b, Bs[buf], kend - k0);
+        }
+    };
+    f32x16 acc = {};
+    // Multiplies the step in buffer `buf`, with the step after the next one
+    // requested into `fut` meanwhile, and moves the next (`nxt`) into LDS.
+    auto step = [&](int buf, const Regs& nxt, Regs& fut, int k0) {
+        if (k0 + 2 * kGK < kend) load(fut, k0 + 2 * kGK);
+        const float* pa = As[buf] + ra * kGS + h4;
+        const float* pb = Bs[buf] + rb * kGS + h4;
+        float4 a[2], b[2];
+        a[0] = *reinterpret_cast<const float4*>(pa);
+        b[0] = *reinterpret_cast<const float4*>(pb);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+        for (int s = 0; s < kGK / 8; ++s) {   // the next eight k's operands are read under these four
+            const int c = s & 1;
+            if (s + 1 < kGK / 8) {
+                a[c ^ 1] = *reinterpret_cast<const float4*>(pa + 8 * (s + 1));
+                b[c ^ 1] = *reinterpret_cast<const float4*>(pb + 8 * (s + 1));
+                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            }
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[c].x, b[c].x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[c].y, b[c].y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[c].z, b[c].z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[c].w, b[c].w, acc, 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+        }
+        if (k0 + kGK < kend) stage(nxt, buf ^ 1, k0 + kGK);
+        __syncthreads();
+    };
+    load(r0, kbeg);
+    if (kbeg + kGK < kend) load(r1, kbeg + kGK);
+    stage(r0, 0, kbeg);
+    __syncthreads();
+    for (int k0 = kbeg; k0 < kend; k0 += 2 * kGK) {
+        step(0, r1, r0, k0);
+        if (k0 + kGK < kend) step(1, r0, r1, k0 + kGK);
+    }
+    // Register r of lane l is row 8(r/4) + 4(l/32) + r%4, column l%32 of the block.
+    const int n = n0 + rb;
+    if (n >= N) return;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int m = m0 + (w / WN) * 32 + 8 * (r >> 2) + h4 + (r & 3);
+        if (m >= M) continue;
+        if (P) {
+            P[((size_t)blockIdx.z * M + m) * N + n] = acc[r];
+        } else {
+            float* c = C + (size_t)m * ldc + n;
+            const float prev = beta == 0.f ? 0.f : (beta == 1.f ? *c : *c * beta);
+            *c = prev + alpha * acc[r];
+        }
+    }
+}
+
+// C = beta*C + alpha * (the S slices' partial sums, in slice order).
+__global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(const float* __restrict__ P, int S, float* C, int M,
+                                                              int N, int ldc, float alpha, float beta) {
+    const size_t mn = (size_t)M * N, i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= mn) return;
+    float v = 0.f;
+    for (int s = 0; s < S; s += 8) {   // eight loads in flight, added in slice order
+        float p[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p[j] = P[min(s + j, S - 1) * mn + i];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v += s + j < S ? p[j] : 0.f;
+    }
+    float* c = C + (i / N) * ldc + i % N;
+    const float prev = beta == 0.f ? 0.f : (beta == 1.f ? *c : *c * beta);
+    *c = prev + alpha * v;
 }
 
 __device__ __forceinline__ float block_sum(float v, float* red) {
@@ -147,15 +269,93 @@ int grid_1d(int64_t n) {
 
 }  // namespace
 
+namespace {
+
+struct GemmF32Plan {
+    bool wide;        // 32 x 128 tiles
+    int S, kslice;    // slices of K, and the columns of one
+};
+
+// The split with the shortest estimated time, in K steps of one tile (about
+// 1.1 us): rounds of 256 workgroups times the steps of a slice, plus, with more
+// than one slice, the reduction: its launch (about 5 steps) and its partial
+// sums at about 3.3 MB a step.  Slices keep at least two steps, and 512 tiles
+// fill the chip twice without a split.  Measured (us, this split against one
+// slice / the next candidates): 300x768x3072 (60 tiles) 23.0 with 4 slices, 38.2
+// with 2, 22.7 with 8; 700x768x3072 (132) 42.6 with 3, 67.8 with 1; 300x3072x768
+// (240) 20.8 with 1, 25.4 with 2; 1x768x3072 (6) 8.6 with 24, 10.6 with 12.
+GemmF32Plan gemm_f32_plan(int M, int N, int K) {
+    GemmF32Plan p;
+    p.wide = M <= 32;
+    const int bm = p.wide ? 32 : 64, bn = p.wide ? 128 : 64;
+    const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    const int steps = (K + kGK - 1) / kGK;
+    int best = 1;
+    if (tiles < 512) {
+        float cost = (float)((tiles + 255) / 256) * steps;
+        for (int S = 2; S <= 64 && S <= steps / 2; ++S) {
+            const float c = (float)((tiles * S + 255) / 256) * ((steps + S - 1) / S) + 5.f +
+                            8e-6f / 3.3f * S * (float)M * N;
+            if (c < cost) {
+                cost = c;
+                best = S;
+            }
+        }
+    }
+    const int per = (steps + best - 1) / best;
+    p.S = (steps + per - 1) / per;
+    p.kslice = per * kGK;
+    return p;
+}
+
+}  // namespace
+
+size_t gemm_f32_part_bytes(int M, int N, int K) {
+    if (M < 1 || N < 1 || K < 1) return 0;
+    const GemmF32Plan p = gemm_f32_plan(M, N, K);
+    return p.S > 1 ? (size_t)p.S * M * N * sizeof(float) : 0;
+}
+
 int launch_gemm_f32(hipStream_t s, const float* A, const float* B, float* C, int M, int N, int K, int lda,
-                    int ldb, int ldc, float alpha, float beta, bool transA, bool transB) {
+                    int ldb, int ldc, float alpha, float beta, bool transA, bool transB, float* part) {
     VH_ARG(A && B && C, "gemm_f32: null operand");
     VH_ARG(M >= 1 && N >= 1 && K >= 1, "gemm_f32: empty shape %dx%dx%d", M, N, K);
     VH_ARG(lda >= (transA ? M : K) && ldb >= (transB ? K : N) && ldc >= N, "gemm_f32: leading dimension too small");
-    dim3 grid((N + kGT - 1) / kGT, (M + kGT - 1) / kGT);
-    hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(256), 0, s, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta,
-                       (int)transA, (int)transB);
+    GemmF32Plan p = gemm_f32_plan(M, N, K);
+    if (!part) {
+        p.S = 1;
+        p.kslice = K;
+    }
+    float* P = p.S > 1 ? part : nullptr;
+    const bool va = ((uintptr_t)A & 15) == 0 && lda % 4 == 0 && lda < (1 << 22) && (transA ? M : K) % 4 == 0;
+    const bool vb = ((uintptr_t)B & 15) == 0 && ldb % 4 == 0 && ldb < (1 << 22) && (transB ? K : N) % 4 == 0;
+    const int bm = p.wide ? 32 : 64, bn = p.wide ? 128 : 64;
+    const dim3 grid((N + bn - 1) / bn, (M + bm - 1) / bm, p.S);
+#define VH_GF(BM, BN, TA, TB, VV)                                                                               \
+    hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, TA, TB, VV>), grid, dim3(256), 0, s, A, B, C, P, M, N, K,    \
+                       lda, ldb, ldc, alpha, beta, p.kslice)
+#define VH_GF_T(BM, BN, VV)                                                                                      \
+    if (transA) {                                                                                                \
+        if (transB) VH_GF(BM, BN, true, true, VV);                                                               \
+        else VH_GF(BM, BN, true, false, VV);                                                                     \
+    } else {                                                                                                     \
+        if (transB) VH_GF(BM, BN, false, true, VV);                                                              \
+        else VH_GF(BM, BN, false, false, VV);                                                                    \
+    }
+    if (p.wide) {
+        if (va && vb) { VH_GF_T(32, 128, true) } else { VH_GF_T(32, 128, false) }
+    } else {
+        if (va && vb) { VH_GF_T(64, 64, true) } else { VH_GF_T(64, 64, false) }
+    }
+#undef VH_GF_T
+#undef VH_GF
     VH_LAUNCHED();
+    if (P) {
+        const size_t mn = (size_t)M * N;
+        hipLaunchKernelGGL(gemm_f32_reduce_kernel, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, s, P, p.S, C, M,
+                           N, ldc, alpha, beta);
+        VH_LAUNCHED();
+    }
     return VLRF_HIP_OK;
 }
 

@@ -28,6 +28,9 @@ struct vlrf_hip_ctx {
     int rope_tables(int max_seq, int d_head, float theta, const float** c, const float** s);
     // Grows the shared scratch buffer (waits for queued work before regrowing).
     int scratch(size_t bytes, float** out);
+    // The same for a caller that can do without: null where it cannot be had
+    // (bytes 0, the stream under capture, no memory).
+    float* try_scratch(size_t bytes);
     ~vlrf_hip_ctx();
 };
 
