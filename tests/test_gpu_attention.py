@@ -47,6 +47,65 @@ def test_sdp_attention_reference_shapes(ctx, orc, T, ctx_len, d, causal, seed):
     assert rel_err(out, ref) <= 1e-3
 
 
+def _sdp64(Q, K, V, scale, causal):
+    """(attention in 64 bits, a bound on an f32 result's distance from it): every
+    weight is off by at most eps ((d + 8) S + 40) relative, S the query's largest
+    |scale| sum |q||k|; the sums over the keys add ctx eps each; both in the
+    numerator and in the normaliser."""
+    n_h, T, d = Q.shape
+    n = K.shape[1]
+    Q, K, V = (t.astype(np.float64) for t in (Q, K, V))
+    keep = np.arange(n)[None, :] <= np.arange(T)[:, None] + (n - T) if causal else np.ones((T, n), bool)
+    s = np.where(keep, Q @ K.transpose(0, 2, 1) * scale, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    S = np.where(keep, np.abs(Q) @ np.abs(K).transpose(0, 2, 1) * abs(scale), 0).max(-1, keepdims=True)
+    return p @ V, 2 * 2.0 ** -24 * ((d + 8) * S + n + 40) * (p @ np.abs(V))
+
+
+@pytest.mark.parametrize("T,ctx_len,d,causal,scale,off", [
+    (1, 1, 1, True, 1.0, 0), (31, 31, 15, True, 0.5, 0), (32, 33, 16, True, 0.25, 0), (33, 64, 17, False, 0.3, 0),
+    (64, 127, 48, True, 0.2, 0), (65, 65, 63, True, 0.125, 0), (40, 129, 64, True, 0.125, 1),   # odd addresses
+    (1, 300, 64, True, 0.125, 0), (100, 100, 80, True, 0.11, 0), (7, 1000, 81, False, 0.11, 0),
+    (50, 34, 96, False, 0.1, 0), (33, 200, 112, True, 0.1, 0), (70, 257, 127, True, 0.09, 0), (97, 97, 128, True, 0.09, 2),
+    (40, 90, 64, True, -0.125, 0), (40, 90, 64, True, 0.0, 0), (5, 2050, 4, False, 0.5, 0)])
+def test_sdp_attention_tiles(ctx, T, ctx_len, d, causal, scale, off):
+    """Edges of the query blocks, key tiles and head-size steps; rows that forbid
+    16-byte loads; negative and zero scales."""
+    print(f"[case] sdp tiles T={T} ctx={ctx_len} d={d} causal={causal} scale={scale} off={off}", flush=True)
+    n_h = 3
+    Q, K, V = _qkv(T * 7 + d, n_h, T, ctx_len, d)
+    bufs = [ctx.to_device(np.concatenate([np.full(off, np.nan, np.float32), t.ravel()])) for t in (Q, K, V)]
+    do = ctx.to_device(np.full(Q.size + 8, 7.0, np.float32))
+    import vlrf_amd as V_
+    V_.check(V_.lib().vlrf_hip_attn_f32(ctx.h, *[b.ptr + 4 * off for b in bufs], do.ptr, n_h, T, ctx_len, d, scale,
+                                        int(causal)))
+    got = do.download((Q.size + 8,))
+    ref, bound = _sdp64(Q, K, V, np.float32(scale), causal)
+    assert (np.abs(got[:Q.size].reshape(Q.shape) - ref) <= bound).all()
+    assert (got[Q.size:] == 7.0).all()
+
+
+def test_sdp_attention_specials(ctx, orc):
+    """-inf scores weigh nothing, a NaN query stays in its row, an infinite value
+    in a key that every query of the block may see reaches all of them."""
+    T, n, d = 40, 200, 64
+    Q, K, V = _qkv(77, 2, T, n, d)
+    Q[0], K[0, 3] = np.abs(Q[0]), -np.inf                     # head 0: key 3 scores -inf
+    Q[1, 5] = np.nan
+    V[1, 0, 2] = np.inf
+    out = _run_gpu(ctx, Q, K, V, np.float32(0.125), True)
+    K0, V0 = np.delete(K[:1], 3, 1), np.delete(V[:1], 3, 1)
+    ref, bound = _sdp64(Q[:1], K0, V0, np.float32(0.125), True)
+    assert (np.abs(out[0] - ref[0]) <= bound[0]).all()
+    cpu = orc.sdp_attention(Q, K, V, np.float32(0.125), True)
+    rows = np.arange(T) != 5
+    assert np.isposinf(out[1][rows, 2]).all() and np.isposinf(cpu[1][rows, 2]).all()
+    fine = np.ones(d, bool)
+    fine[2] = False
+    assert rel_err(out[1][rows][:, fine], cpu[1][rows][:, fine]) <= 1e-3
+
+
 def test_config1_decode_f32(ctx, orc):
     """Benchmark config 1: 1 query, 8 heads, d 64, KV 512, non-causal, scale 1/8."""
     Q, K, V = _qkv(11, 8, 1, 512, 64)

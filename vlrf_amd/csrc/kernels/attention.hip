@@ -44,6 +44,7 @@ constexpr int kChunk = 64;        // tokens per split-K workgroup
 constexpr int kAttnThreads = 512;  // lanes per decode-attention workgroup (8 waves)
 constexpr int kMaxSplits = 512;   // contexts up to 32768 tokens
 constexpr float kNegInf = -INFINITY;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 using attn::rope2;
 
@@ -632,7 +633,6 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(
     float scale, int n_heads, const float* __restrict__ cos_t, const float* __restrict__ sin_t,
     uint16_t* __restrict__ out) {
     typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-    typedef float f32x16 __attribute__((ext_vector_type(16)));
     constexpr int NT = 512, NQB = 8 / REP;           // waves: REP heads x NQB query blocks
     constexpr int KS = D + 8, VS = kPK + 8;          // padded LDS row strides (bf16)
     constexpr int ITEMS = kPK * (D / 16);            // staging items of 16 elements per tile
@@ -856,84 +856,200 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(
     }
 }
 
-// ---- general f32 attention: one thread per query row, 64x64 tiles --------------
-template <int D>
-__global__ __launch_bounds__(64) void attn_f32_tiled_kernel(const float* __restrict__ Q,
-                                                            const float* __restrict__ K,
-                                                            const float* __restrict__ V,
-                                                            float* __restrict__ O, int T, int ctx,
-                                                            int d, float scale, int causal) {
-    __shared__ __align__(16) float Kt[64][D];
-    __shared__ __align__(16) float Vt[64][D];
-    const int h = blockIdx.y, q0 = blockIdx.x * 64, lane = threadIdx.x, qi = q0 + lane;
-    const float* Qh = Q + (size_t)h * T * d;
+// ---- general f32 attention ---------------------------------------------------------
+// flash_attn_head (attention.hpp:207-309) over f32 Q/K/V on the f32 matrix
+// instructions.  A workgroup owns one head's block of 32 queries; its four
+// waves take the 32-key tiles in turn, each with its own online softmax, and
+// merge (m, l, O) through LDS at the end in wave order.
+// S^T = K.Q^T puts a query's 32 scores into two lanes (lane l: query l % 32, keys
+// 8(r/4) + 4(l/32) + r%4 in register r), which are then the B operand of
+// O^T = V^T.P^T as they are: no exchange between the products but the maximum's.
+// Operands come straight from memory (buffer loads: per-tile resources, so the
+// addresses cost no vector instructions): lane half h takes a K row's dims
+// 8s + 4h + 0..3 (the order of the dims is the same for q), V rows are read 32
+// consecutive dims a half.  V's loads are in flight under the first product and
+// the softmax, the next K tile's under the softmax and the second.
+//
+// Bound by the matrix rate and, beside it, the softmax's vector work (about 300
+// instructions to the 64 matrix instructions of a tile at d 64, two waves a
+// SIMD).  Measured against one thread a query on the vector units (32 heads, d
+// 64, causal): 777 x 777 keys 766 -> 41 us, 1024 x 1024 997 -> 54 (79
+// TFLOP/s); d 128, 1024 x 2048 keys 7205 -> 286; 12 heads, 41 x 568 474 -> 15.
+// Plain 64-bit addresses ran 64.6, these loads 41; eight waves a block 44.6.
+//
+// Weights are exp2(s * sl2 - m * sl2) with one rounding at the difference's
+// size and the scores' sums run in two chains: the error against 64 bits over
+// these shapes is at or below the vector kernel's (3.4e-7 against 4.0e-7 at 777).
+//
+// DP: d rounded up to 16, zeros beyond d in both q and K.  VEC: 16-byte loads
+// (d % 4 == 0, aligned bases).  Masked keys weigh 0; as in the reference's
+// 64-key blocks, a non-finite V value of a masked key reaches the queries of
+// its tile (0 * inf).
+// Rows of 32 keys from a tile's own buffer resource: rows past the head's last
+// key are past its end and read as zeros.
+template <int NS, bool VEC>
+__device__ __forceinline__ void f32_row(float4 (&v)[NS], __amdgpu_buffer_rsrc_t rs, int row, int hh, int d) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        const int i = 8 * s + 4 * hh;
+        if constexpr (VEC) {
+            v[s] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, 4 * (row * d + min(i, d - 4)), 0, 0));
+        } else {
+            float x[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                x[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, 4 * (row * d + min(i + j, d - 1)), 0, 0));
+            v[s] = make_float4(x[0], x[1], x[2], x[3]);
+        }
+    }
+}
+
+template <int NS>
+__device__ __forceinline__ void f32_row_zero_past(float4 (&v)[NS], int hh, int d) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        const int i = 8 * s + 4 * hh;
+        v[s].x = i < d ? v[s].x : 0.f;
+        v[s].y = i + 1 < d ? v[s].y : 0.f;
+        v[s].z = i + 2 < d ? v[s].z : 0.f;
+        v[s].w = i + 3 < d ? v[s].w : 0.f;
+    }
+}
+
+template <int DP, bool VEC>
+__global__ __launch_bounds__(256, DP <= 64 ? 2 : 1) void attn_f32_mfma_kernel(
+    const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V, float* __restrict__ O, int T,
+    int ctx, int d, float sl2, float qsign, int causal) {
+    constexpr int NS = DP / 8, NC = (DP + 31) / 32, OS = 32 * NC + 4, NW = 4;
+    __shared__ __align__(16) float os[NW][32 * OS];   // a wave's O by query
+    __shared__ float ms[NW][32], ls[NW][32];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: so are the tiles
+    const int lq = lane & 31, hh = lane >> 5;
+    const int h = blockIdx.x, q0 = 32 * (int)(gridDim.y - 1 - blockIdx.y);   // the longest causal rows first
     const float* Kh = K + (size_t)h * ctx * d;
     const float* Vh = V + (size_t)h * ctx * d;
-    float qv[D], acc[D];
-#pragma unroll
-    for (int i = 0; i < D; ++i) {
-        qv[i] = (qi < T && i < d) ? Qh[(size_t)qi * d + i] : 0.f;
-        acc[i] = 0.f;
-    }
-    float m = kNegInf, l = 0.f;
-    const int past = ctx - T;
-    const int br = min(64, T - q0);
-    const int k_limit = causal ? min(ctx, q0 + br + past) : ctx;
-    const int qpos = qi + past;
+    const int past = ctx - T, qpos = q0 + lq + past;
+    const int k_limit = causal ? min(ctx, q0 + 32 + past) : ctx;
+    const int ntile = (k_limit + 31) / 32;
 
-    for (int k0 = 0; k0 < k_limit; k0 += 64) {
-        const int bc = min(64, k_limit - k0);
-        for (int i = lane; i < 64 * D; i += 64) {
-            const int r = i / D, c = i % D;
-            const bool ok = r < bc && c < d;
-            Kt[r][c] = ok ? Kh[(size_t)(k0 + r) * d + c] : 0.f;
-            Vt[r][c] = ok ? Vh[(size_t)(k0 + r) * d + c] : 0.f;
+    auto tile = [&](const float* X, int t, int rows) {
+        const int n = min(32, rows - 32 * t);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(X + (size_t)32 * t * d), 0, n * d * 4, 0x00020000);
+    };
+    float4 qv[NS], kv[NS];
+    f32_row<NS, VEC>(qv, tile(Q + (size_t)h * T * d, q0 / 32, T), lq, hh, d);
+    const int first = (w + h + (int)blockIdx.y) % NW;   // the odd tiles fall to another SIMD in each workgroup
+    f32_row<NS, VEC>(kv, tile(Kh, min(first, ntile - 1), k_limit), lq, hh, d);
+    f32_row_zero_past<NS>(qv, hh, d);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) qv[s] = make_float4(qsign * qv[s].x, qsign * qv[s].y, qsign * qv[s].z, qsign * qv[s].w);
+    int vo[NC];   // the lane's V elements: dims 32c + lq of row 4hh
+#pragma unroll
+    for (int c = 0; c < NC; ++c) vo[c] = 4 * (4 * hh * d + min(32 * c + lq, d - 1));
+
+    f32x16 o[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) o[c] = f32x16{};
+    // m: the largest score so far (before the scale), m2 = m * sl2 (0 while there
+    // is none); l: this half's keys.
+    float m = kNegInf, m2 = 0.f, l = 0.f;
+    for (int t = first; t < ntile; t += NW) {
+        const int k0 = 32 * t;
+        const __amdgpu_buffer_rsrc_t vr = tile(Vh, t, k_limit);
+        float vv[NC][16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                vv[c][r] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_raw_buffer_load_b32(vr, vo[c] + 4 * (8 * (r >> 2) + (r & 3)) * d, 0, 0));
+        if (DP > d) f32_row_zero_past<NS>(kv, hh, d);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x16 s = {}, s1 = {};   // two chains: half the roundings in a row
+#pragma unroll
+        for (int i = 0; i < NS; i += 2) {
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].x, qv[i].x, s, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i + 1].x, qv[i + 1].x, s1, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].y, qv[i].y, s, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i + 1].y, qv[i + 1].y, s1, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].z, qv[i].z, s, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i + 1].z, qv[i + 1].z, s1, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].w, qv[i].w, s, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i + 1].w, qv[i + 1].w, s1, 0, 0, 0);
         }
-        __syncthreads();
-        for (int j0 = 0; j0 < bc; j0 += 16) {
-            float s[16], bmax = kNegInf;
+        f32_row<NS, VEC>(kv, tile(Kh, min(t + NW, ntile - 1), k_limit), lq, hh, d);
+        __builtin_amdgcn_sched_barrier(0);
+        s += s1;
+        // Keys past the query's last one weigh 0: only tiles that reach past the
+        // block's first query's last key hold any.
+        const bool edge = k0 + 31 > (causal ? min(q0 + past, k_limit - 1) : k_limit - 1);
+        const int live = (causal ? min(qpos, k_limit - 1) : k_limit - 1) - k0 - 4 * hh;
+        float mt = kNegInf;
+        if (edge) {
 #pragma unroll
-            for (int jj = 0; jj < 16; ++jj) {
-                const int j = j0 + jj;
-                float dot = 0.f;
+            for (int r = 0; r < 16; ++r) mt = fmaxf(mt, 8 * (r >> 2) + (r & 3) <= live ? s[r] : kNegInf);
+        } else {
 #pragma unroll
-                for (int i = 0; i < D; i += 4) {
-                    const float4 kv = *reinterpret_cast<const float4*>(&Kt[j][i]);
-                    dot += qv[i] * kv.x + qv[i + 1] * kv.y + qv[i + 2] * kv.z + qv[i + 3] * kv.w;
-                }
-                float sj = dot * scale;
-                if (j >= bc || (causal && k0 + j > qpos)) sj = kNegInf;
-                s[jj] = sj;
-                bmax = fmaxf(bmax, sj);
-            }
-            if (bmax != kNegInf) {
-                const float m_new = fmaxf(m, bmax);
-                float bsum = 0.f;
-#pragma unroll
-                for (int jj = 0; jj < 16; ++jj) { s[jj] = expf(s[jj] - m_new); bsum += s[jj]; }
-                const float corr = (m == kNegInf) ? 0.f : expf(m - m_new);
-                l = l * corr + bsum;
-#pragma unroll
-                for (int i = 0; i < D; ++i) acc[i] *= corr;
-#pragma unroll
-                for (int jj = 0; jj < 16; ++jj) {
-                    const float p = s[jj];
-#pragma unroll
-                    for (int i = 0; i < D; i += 4) {
-                        const float4 vv = *reinterpret_cast<const float4*>(&Vt[j0 + jj][i]);
-                        acc[i] += p * vv.x; acc[i + 1] += p * vv.y;
-                        acc[i + 2] += p * vv.z; acc[i + 3] += p * vv.w;
-                    }
-                }
-                m = m_new;
-            }
+            for (int r = 0; r < 16; ++r) mt = fmaxf(mt, s[r]);
         }
-        __syncthreads();
+        const float2 both = swap_halves32(mt, mt);
+        const float mn = fmaxf(m, fmaxf(both.x, both.y));
+        const float m2n = mn == kNegInf ? 0.f : mn * sl2;
+        const float corr = m == kNegInf ? 0.f : __builtin_amdgcn_exp2f(m2 - m2n);
+        float p[16], sum = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], sl2, -m2n));
+        if (edge) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) p[r] = 8 * (r >> 2) + (r & 3) <= live ? p[r] : 0.f;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum += p[r];
+        l = l * corr + sum;
+        if (__builtin_amdgcn_ballot_w64(m != mn)) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[c][r] *= corr;
+        }
+        m = mn;
+        m2 = m2n;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) o[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[c][r], p[r], o[c], 0, 0, 0);
     }
-    if (qi < T) {
-        const float inv = (l > 0.f) ? 1.f / l : 0.f;
-        float* Oh = O + (size_t)h * T * d + (size_t)qi * d;
-        for (int i = 0; i < d; ++i) Oh[i] = acc[i] * inv;
+
+    const float2 lb = swap_halves32(l, l);
+    if (hh == 0) {
+        ms[w][lq] = m == kNegInf ? kNegInf : m2;
+        ls[w][lq] = lb.x + lb.y;
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int a = 0; a < 4; ++a)   // register 4a + j of block c: dim 32c + 8a + 4hh + j
+            *reinterpret_cast<float4*>(&os[w][lq * OS + 32 * c + 8 * a + 4 * hh]) =
+                make_float4(o[c][4 * a], o[c][4 * a + 1], o[c][4 * a + 2], o[c][4 * a + 3]);
+    __syncthreads();
+    constexpr int TPQ = 2 * NW;   // threads per query
+    const int q = threadIdx.x / TPQ, part = threadIdx.x % TPQ;
+    if (q0 + q >= T) return;
+    float M = ms[0][q], f[NW], L = 0.f;
+#pragma unroll
+    for (int i = 1; i < NW; ++i) M = fmaxf(M, ms[i][q]);
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        f[i] = ms[i][q] == kNegInf ? 0.f : __builtin_amdgcn_exp2f(ms[i][q] - M);
+        L += f[i] * ls[i][q];
+    }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    float* Oq = O + ((size_t)h * T + q0 + q) * d;
+    for (int i = part; i < d; i += TPQ) {
+        float x = 0.f;
+#pragma unroll
+        for (int j = 0; j < NW; ++j) x += f[j] * os[j][q * OS + i];
+        Oq[i] = x * inv;
     }
 }
 
@@ -1360,14 +1476,27 @@ int launch_attn_f32_tiled(hipStream_t s, const float* Q, const float* K, const f
     VH_ARG(n_h >= 1 && T >= 1 && ctx_len >= 1, "attn_f32: empty shape");
     VH_ARG(d_h >= 1 && d_h <= 128, "attn_f32: d_h %d outside [1,128]", d_h);
     VH_ARG(T <= ctx_len || !causal, "attn_f32: causal with T > ctx_len");
-    dim3 grid((T + 63) / 64, n_h), block(64);
-#define VH_AT(D) hipLaunchKernelGGL((attn_f32_tiled_kernel<D>), grid, block, 0, s, Q, K, V, O, T, \
-                                    ctx_len, d_h, scale, causal)
-    if (d_h <= 8) VH_AT(8);
-    else if (d_h <= 16) VH_AT(16);
-    else if (d_h <= 32) VH_AT(32);
-    else if (d_h <= 64) VH_AT(64);
-    else VH_AT(128);
+    const bool vec = d_h % 4 == 0 && (((uintptr_t)Q | (uintptr_t)K) & 15) == 0;
+    const dim3 grid(n_h, (T + 31) / 32);   // a head's workgroups on one XCD when 8 divides the heads: its K/V in one L2
+    // Scores in powers of 2; a negative scale's sign goes to q, so that the largest score stays the largest.
+    const float sl2 = (float)(std::fabs((double)scale) * 1.4426950408889634), qsign = scale < 0.f ? -1.f : 1.f;
+#define VH_AT(DP)                                                                                              \
+    if (vec)                                                                                                   \
+        hipLaunchKernelGGL((attn_f32_mfma_kernel<DP, true>), grid, dim3(256), 0, s, Q, K, V, O, T, ctx_len, d_h, \
+                           sl2, qsign, causal);                                                                \
+    else                                                                                                       \
+        hipLaunchKernelGGL((attn_f32_mfma_kernel<DP, false>), grid, dim3(256), 0, s, Q, K, V, O, T, ctx_len,   \
+                           d_h, sl2, qsign, causal)
+    switch ((d_h + 15) / 16) {
+        case 1: VH_AT(16); break;
+        case 2: VH_AT(32); break;
+        case 3: VH_AT(48); break;
+        case 4: VH_AT(64); break;
+        case 5: VH_AT(80); break;
+        case 6: VH_AT(96); break;
+        case 7: VH_AT(112); break;
+        default: VH_AT(128); break;
+    }
 #undef VH_AT
     VH_LAUNCHED();
     return VLRF_HIP_OK;
