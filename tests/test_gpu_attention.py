@@ -213,3 +213,45 @@ def test_decode_attention_chunk_sizes(ctx, orc, kv_name, n_heads, n_kv, ctx_len)
                               for h in range(n_heads)])
         assert rel_err(out, ref) <= 1e-3, (call, n)
         assert np.max(np.abs(out - ref)) <= 1e-4, (call, n)
+
+
+@pytest.mark.parametrize("kv_name", ["Q8_0", "F16", "F32"])
+@pytest.mark.parametrize("n_heads,n_kv,d,ctx_len,scale", [
+    (4, 4, 128, 1, 0.1), (8, 8, 128, 63, 0.1), (8, 4, 128, 64, 0.1), (8, 2, 128, 65, 0.1), (16, 2, 128, 255, 0.1),
+    (8, 8, 128, 256, 0.1), (32, 8, 128, 257, 0.1), (16, 4, 128, 1023, -0.1), (8, 1, 128, 4097, 0.1),
+    (32, 8, 128, 6001, 0.1), (8, 8, 64, 8193, 0.125), (16, 8, 64, 8200, 0.0), (32, 4, 64, 8197, 0.125),
+    (32, 8, 64, 4200, 0.125)])   # 8.6 MB of K/V at Q8_0 is past the one-launch form only in f16 and f32
+def test_decode_attention_rows(ctx, kv_name, n_heads, n_kv, d, ctx_len, scale):
+    """d_head 128, long contexts and large caches: edges of the rounds, of the
+    chunks and of the single-chunk form; all GQA groups; rows past the context
+    that hold infinities; the call that allocates nothing gives the same bits."""
+    import vlrf_amd as V_
+    dt = {"Q8_0": V_.KV_Q8_0, "F16": V_.KV_F16, "F32": V_.KV_F32}[kv_name]
+    print(f"[case] decode rows kv={kv_name} heads={n_heads}/{n_kv} d={d} ctx={ctx_len} scale={scale}", flush=True)
+    row, more = n_kv * d, 40
+    K, V = (F.normal(21, f"{n}{ctx_len}", (ctx_len + more) * row).reshape(-1, row) for n in "kv")
+    if dt != V_.KV_Q8_0:
+        K[ctx_len:], V[ctx_len:] = np.nan, np.inf
+    kv = V_.KVCache(ctx, 2, ctx_len + more, n_kv, d, dt)
+    kv.append(1, ctx.to_device(K), ctx.to_device(V), ctx_len + more)
+    Kd, Vd = (t[:ctx_len].reshape(ctx_len, n_kv, d).transpose(1, 0, 2).repeat(n_heads // n_kv, 0)
+              for t in _dequant_rows_of(kv, 1, ctx_len + more))
+    q = F.normal(22, f"q{ctx_len}", n_heads * d)
+    dq, dout, dfix = ctx.to_device(q), ctx.alloc(q.nbytes), ctx.alloc(q.nbytes)
+    kv.attention_decode(1, dq, dout, n_heads, ctx_len, scale)
+    out = dout.download((n_heads, d))
+    ref, bound = _sdp64(q.reshape(n_heads, 1, d), Kd, Vd, np.float32(scale), False)
+    assert (np.abs(out - ref[:, 0]) <= bound[:, 0]).all()
+    if n_heads * ((ctx_len + 63) // 64) * (d + 2) <= 1 << 19:
+        V_.check(V_.lib().vlrf_hip_attn_decode_noalloc(kv.h, 1, dq.ptr, dfix.ptr, n_heads, ctx_len, float(scale)))
+        assert np.array_equal(dfix.download((n_heads, d)), out)
+
+
+def _dequant_rows_of(kv, layer, n):
+    import vlrf_amd as V_
+    kq, vq, ks, vs = kv.read(layer, 0, n)
+    if kv.dtype == V_.KV_Q8_0:
+        return kq.astype(np.float32) * ks[:, None], vq.astype(np.float32) * vs[:, None]
+    if kv.dtype == V_.KV_F16:
+        return kq.view(np.float16).astype(np.float32), vq.view(np.float16).astype(np.float32)
+    return kq, vq

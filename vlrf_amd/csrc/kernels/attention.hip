@@ -20,17 +20,19 @@
 // (m, l, acc[d]) per (head, chunk) are merged by a combine kernel with the
 // log-sum-exp rescale.  With a device-side position the kernel also applies
 // RoPE to q and to the new k and quantizes + stores the new K/V row before
-// attending (the decode step's fused form).
+// attending: it always runs as the decode step's fused form.
 //
 // The decode step itself (d_head 64, caches of 513..8192 rows) runs the
 // single-pass kernel below in chunked form instead: one query head and one
 // 512-row chunk per workgroup, a (m, l, acc) partial per chunk, merged by the
 // O projection's GEMV prologue, so the step has no combine launch; caches of
 // at most 512 rows take the single pass over the whole context.  The
-// stand-alone calls (vlrf_hip_attn_decode, vlrf_hip_attn_f32 at T = 1) at
-// d_head 64 run attn_decode_chunks_kernel: the same chunk code on 64..512-row
-// chunks, merged in the same launch by each head's last workgroup; the
-// split-K kernel and its combine serve d_head 128 and longer contexts.
+// stand-alone calls (vlrf_hip_attn_decode, vlrf_hip_attn_f32 at T = 1) run
+// attn_decode_chunks_kernel at d_head 64 while the K/V are small (the same chunk
+// code on 64..512-row chunks, merged in the same launch by each head's last
+// workgroup), else attn_decode_rows_kernel and its merge; the split-K kernel and
+// its combine serve the step's other forms (d_head 128 beside the chunked one,
+// longer caches).
 #include "../internal.hpp"
 #include "attn_core.hpp"
 
@@ -51,10 +53,10 @@ using attn::rope2;
 // KVT: cache element type VLRF_HIP_KV_Q8_0 (int8 codes, f32 scale per token row),
 // VLRF_HIP_KV_F16 (the reference's f16 bits) or VLRF_HIP_KV_F32; kc/vc address the
 // elements ([n_kv][head_stride/D][D]) as bytes.
-template <int D, int REP, int KVT, bool FUSED>
+template <int D, int REP, int KVT>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_partial_kernel(
     const float* __restrict__ q, const int8_t* kc, const int8_t* vc, const float* ks, const float* vs,
-    long head_stride, int ctx_len, const int* __restrict__ ctx_dev, int n_splits, float scale,
+    long head_stride, const int* __restrict__ ctx_dev, int n_splits, float scale,
     float* __restrict__ part, DecodeFuse fz) {
     constexpr bool Q8 = KVT == VLRF_HIP_KV_Q8_0, H16 = KVT == VLRF_HIP_KV_F16;
     constexpr int EB = Q8 ? 1 : H16 ? 2 : 4;             // bytes per cache element
@@ -71,8 +73,8 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_partial_kernel(
     __shared__ __align__(16) float vsm[kChunk][D];       // the chunk's dequantized V rows
     __shared__ __align__(16) float pr[REP][kChunk];      // softmax numerators
     __shared__ float mstat[REP], lstat[REP];
-    __shared__ __align__(16) float newk[FUSED ? D : 1];
-    __shared__ float amax[FUSED ? 2 * NW : 1];          // per-wave maxima of the new K and V rows
+    __shared__ __align__(16) float newk[D];
+    __shared__ float amax[2 * NW];                     // per-wave maxima of the new K and V rows
 
     const int split = blockIdx.x, g = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -97,7 +99,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_partial_kernel(
     // Fused decode: the new token's row spread over the workgroup (rows of at
     // most 1024 elements): thread t holds K RoPE pair t and V elements t, t + NT.
     float nk0 = 0.f, nk1 = 0.f, nv0 = 0.f, nv1 = 0.f;
-    if constexpr (FUSED) {
+    {
         const int npairs = fz.n_kv * HALF, nrow = fz.n_kv * D;
         const int i = min(tid, npairs - 1), h = i / HALF, j = i - h * HALF;
         nk0 = fz.k_new[h * D + j];
@@ -124,12 +126,11 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_partial_kernel(
 
     // The device position is read only now: none of the addresses above depend
     // on it, so its latency overlaps the cache stream.
-    const int dpos = (FUSED || ctx_dev) ? *ctx_dev : 0;   // fused: always a device position
-    int ctx = FUSED ? dpos + 1 : (ctx_dev ? dpos + ctx_len : ctx_len);   // FUSED: dpos = tokens before this one
+    const int pos = *ctx_dev;   // tokens before this one
+    int ctx = pos + 1;
     // Rows past the cache capacity are never read, even if the device-side
     // position were corrupt (the host checks capacity before queuing).
     ctx = min(ctx, cap);
-    const int pos = FUSED ? dpos : -1;
     float* pout = part + (size_t)(g * REP) * n_splits * (D + 2) + (size_t)split * (D + 2);
     if (c0 >= ctx) {   // chunk past the context: empty partial
         for (int i = tid; i < REP * (D + 2); i += NT) {
@@ -139,13 +140,13 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_partial_kernel(
         return;
     }
     const int nt = min(kChunk, ctx - c0);       // valid tokens of the chunk
-    const bool has_new = FUSED && pos >= c0 && pos < c0 + kChunk;
-    const bool rot = FUSED && pos < fz.max_seq;   // rope.hpp:84: positions >= max_seq stay unrotated
+    const bool has_new = pos >= c0 && pos < c0 + kChunk;
+    const bool rot = pos < fz.max_seq;   // rope.hpp:84: positions >= max_seq stay unrotated
     // Every RoPE pair this thread rotates (q pairs tid + NT*p, and for wave 0
     // the new k pairs lane + 64p) has pair index tid % HALF, so one table entry
     // per thread serves them all.
     float rc = 1.f, rs = 0.f;
-    if constexpr (FUSED) {
+    {
         const int trow = min(pos, fz.max_seq - 1);   // used only when rot
         rc = fz.cos_t[(size_t)trow * HALF + (tid & (HALF - 1))];
         rs = fz.sin_t[(size_t)trow * HALF + (tid & (HALF - 1))];
@@ -206,8 +207,8 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_partial_kernel(
     // work (one pair and up to two V elements per thread): the row maxima are
     // wave reductions merged through LDS at the barrier below, so the chain
     // before the scores is a few dozen instructions long.
-    const int npairs = FUSED ? fz.n_kv * HALF : 0, nrow = FUSED ? fz.n_kv * D : 0;
-    if constexpr (FUSED) {
+    const int npairs = fz.n_kv * HALF, nrow = fz.n_kv * D;
+    {
         if (has_new) {
             if (tid < npairs && rot) rope2(nk0, nk1, rc, rs, &nk0, &nk1);
             if constexpr (Q8) {
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_partial_kernel(
     // for the store as well.
     uint32_t kb0 = 0, kb1 = 0, vb0 = 0, vb1 = 0;
     float sk = 1.f, sv = 1.f;
-    if constexpr (FUSED) {
+    {
         if (has_new) {
             float ak = 0.f, av = 0.f, ik = 0.f, iv = 0.f;
             if constexpr (Q8) {
@@ -291,7 +292,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_partial_kernel(
                 for (int k = 0; k < 4; ++k) kv[4 * i + k] = __uint_as_float(w[k]);
             }
         }
-        if constexpr (FUSED) {
+        {
             if (has_new && c0 + lane == pos) {     // the new token: its stored row, as read back
 #pragma unroll
                 for (int j = 0; j < D; ++j) kv[j] = newk[j];
@@ -351,7 +352,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_partial_kernel(
         pout[(size_t)tid * n_splits * (D + 2) + D + 1] = lstat[tid];
     }
     // ---- fused: the new row into the cache (head g's elements; KV head 0 the scales)
-    if constexpr (FUSED) {
+    {
         if (has_new) {
             int8_t* krow_w = fz.kq_w + (hb + (size_t)pos * D) * EB;
             int8_t* vrow_w = fz.vq_w + (hb + (size_t)pos * D) * EB;
@@ -407,12 +408,12 @@ constexpr int kCH = 512, kChunkStride = kAttnChunkStride;   // 256 / 1024: 0.645
 // cache per workgroup, NW = CH/64 waves of one round, for query head h of
 // chunk s; the result is the chunk's partial (m, l, acc) at out[h][s][*]
 // (kChunkStride floats), the new token merged only by the chunk holding it.
-template <int KVT, int REP, bool FUSED, int CH = 0>
+template <int KVT, int REP, int CH = 0>
 __global__ __launch_bounds__(CH ? CH : 64 * kSPWaves) void attn_decode_single_kernel(
     const float* __restrict__ q, const int8_t* kc, const int8_t* vc, const float* ks, const float* vs,
-    long head_stride, int ctx_len, const int* __restrict__ ctx_dev, float scale, float* __restrict__ out,
+    long head_stride, const int* __restrict__ ctx_dev, float scale, float* __restrict__ out,
     DecodeFuse fz, int nch) {
-    static_assert(CH == 0 || (FUSED && CH % 64 == 0), "chunks: fused decode, whole rounds");
+    static_assert(CH % 64 == 0, "chunks: whole rounds");
     static_assert(kSPRounds == 1 && kSPDepth == 1, "attn::chunk runs one round per wave");
     constexpr int D = attn::D, HALF = attn::HALF, NW = CH ? CH / 64 : kSPWaves;
     __shared__ attn::Smem<NW> sm;
@@ -448,7 +449,7 @@ __global__ __launch_bounds__(CH ? CH : 64 * kSPWaves) void attn_decode_single_ke
     // RoPE pair t and V elements t and (with 256 threads) t + NT.
     constexpr int NT = 64 * NW;
     attn::NewRow nr;
-    if constexpr (FUSED) {
+    {
         const int npairs = fz.n_kv * HALF, nrow = fz.n_kv * D;
         const int i = min(tid, npairs - 1), hh = i / HALF, j = i - hh * HALF;
         nr.k0 = fz.k_new[hh * D + j];
@@ -463,18 +464,17 @@ __global__ __launch_bounds__(CH ? CH : 64 * kSPWaves) void attn_decode_single_ke
     // lands between the K and the V loads.
     __builtin_amdgcn_sched_barrier(0);
 
-    const int dpos = (FUSED || ctx_dev) ? *ctx_dev : 0;   // fused: always a device position
-    int ctx = FUSED ? dpos + 1 : (ctx_dev ? dpos + ctx_len : ctx_len);
+    const int pos = *ctx_dev;   // tokens before this one
+    int ctx = pos + 1;
     ctx = min(ctx, cap);
-    const int pos = FUSED ? dpos : -1;
-    const bool rot = FUSED && pos < fz.max_seq;      // rope.hpp:84: positions >= max_seq stay unrotated
-    const bool has_new = FUSED && (CH == 0 || (pos >= c0 && pos < c0 + CH));
-    if constexpr (FUSED) attn::rope_row(nr, fz, pos);
+    const bool rot = pos < fz.max_seq;      // rope.hpp:84: positions >= max_seq stay unrotated
+    const bool has_new = (CH == 0 || (pos >= c0 && pos < c0 + CH));
+    attn::rope_row(nr, fz, pos);
     // A chunk past the context takes no early exit: it runs no round and the merge
     // writes its empty partial (acc 0, m -inf, l 0).  An exit on the device
     // position here lets the compiler sink the K/V loads below that position's
     // load, adding its round trip to every workgroup.
-    attn::chunk<KVT, FUSED, NW>(sm, R, q0, q1, nr, h % REP == 0, h == 0, g, c0, cap, hb, ctx, pos, rot, has_new, scale, fz,
+    attn::chunk<KVT, true, NW>(sm, R, q0, q1, nr, h % REP == 0, h == 0, g, c0, cap, hb, ctx, pos, rot, has_new, scale, fz,
                                 [&](int t, float ot, float mt, float lt) {
                                     if constexpr (CH > 0) {   // the chunk's partial, unnormalised
                                         float* pp = out + ((size_t)h * nch + chunk) * kChunkStride;
@@ -1195,6 +1195,296 @@ __global__ __launch_bounds__(kCH) void attn_chunk128_kernel(const float* __restr
 }
 
 
+// ---- stand-alone decode attention over long contexts and d_head 128 ---------------
+// A workgroup of four waves owns up to four query heads of one KV head and a
+// chunk of the context, so each K/V byte is read once for them.  A wave's load
+// instruction covers 1 KiB of consecutive rows: LPR = D / EPL lanes a row, EPL
+// elements (16 bytes) a lane.  A round is eight such loads of K and of V, the
+// next round's in flight; rows past the context are past the round's buffer
+// resource and read as zeros.  A lane multiplies its dims with each head's q (in
+// registers), the LPR lanes of a row add up (DPP), so every lane of a row holds
+// its score and, after the wave's common maximum, its weight: P.V needs no
+// exchange, and the rows' lanes are added once, after the last round.  Weights
+// are exp2(s * sl2 - m * sl2), one rounding at the difference's size.  Partials
+// (acc[D], m * sl2, l) per head and chunk, merged by attn_decode_merge_kernel; a
+// single chunk is the result.
+template <int LPR>
+__device__ __forceinline__ float row_sum(float v) {   // over the LPR lanes of a row
+    v += dpp_f<0xB1>(v);
+    v += dpp_f<0x4E>(v);
+    if constexpr (LPR >= 8) v += dpp_f<0x141>(v);
+    if constexpr (LPR >= 16) v += dpp_f<0x140>(v);
+    if constexpr (LPR >= 32) {
+        const float2 t = swap_rows16(v, v);
+        v = t.x + t.y;
+    }
+    return v;
+}
+
+template <int LPR, bool MAX>
+__device__ __forceinline__ float across_rows(float v) {   // over the rows of a load, the lanes of one alike
+    auto op = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
+    if constexpr (LPR < 8) v = op(v, dpp_f<0x141>(v));
+    if constexpr (LPR < 16) v = op(v, dpp_f<0x140>(v));
+    if constexpr (LPR < 32) {
+        const float2 t = swap_rows16(v, v);
+        v = op(t.x, t.y);
+    }
+    const float2 t = swap_halves32(v, v);
+    return op(t.x, t.y);
+}
+
+// The lanes of a row hold different dims: add lanes a multiple of LPR apart.
+template <int LPR>
+__device__ __forceinline__ float across_rows_dims(float v) {
+    if constexpr (LPR < 8) v += dpp_f<0x124>(v);    // rotate by 4, then (below) by 8: all four
+    if constexpr (LPR < 16) v += dpp_f<0x128>(v);
+    if constexpr (LPR < 32) {
+        const float2 t = swap_rows16(v, v);
+        v = t.x + t.y;
+    }
+    const float2 t = swap_halves32(v, v);
+    return t.x + t.y;
+}
+
+template <int KVT>
+__device__ __forceinline__ void words_f32(const uint4& k, float (&f)[KVT == VLRF_HIP_KV_Q8_0 ? 16 : KVT == VLRF_HIP_KV_F16 ? 8 : 4]) {
+    const uint32_t u[4] = {k.x, k.y, k.z, k.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (KVT == VLRF_HIP_KV_Q8_0) {
+            const float4 x = attn::s8f4(u[i]);
+            f[4 * i] = x.x; f[4 * i + 1] = x.y; f[4 * i + 2] = x.z; f[4 * i + 3] = x.w;
+        } else if constexpr (KVT == VLRF_HIP_KV_F16) {
+            f[2 * i] = f16_bits_to_f32(u[i] & 0xFFFFu);
+            f[2 * i + 1] = f16_bits_to_f32(u[i] >> 16);
+        } else {
+            f[i] = __uint_as_float(u[i]);
+        }
+    }
+}
+
+template <int D, int KVT, int NL_>
+struct RowsCfg {
+    static constexpr int EB = KVT == VLRF_HIP_KV_Q8_0 ? 1 : KVT == VLRF_HIP_KV_F16 ? 2 : 4;
+    static constexpr int EPL = 16 / EB, LPR = D / EPL, RPL = 64 / LPR, NL = NL_, RR = NL * RPL;   // RR: rows a round
+};
+
+template <int D, int HG, int KVT, int NL_>
+__global__ __launch_bounds__(256) void attn_decode_rows_kernel(
+    const float* __restrict__ q, const int8_t* kc, const int8_t* vc, const float* ks, const float* vs,
+    long head_stride, int ctx, int rep, int rounds, float sl2, float qsign, float* __restrict__ part,
+    float* __restrict__ out) {
+    using C = RowsCfg<D, KVT, NL_>;
+    constexpr bool Q8 = KVT == VLRF_HIP_KV_Q8_0;
+    constexpr int EPL = C::EPL, LPR = C::LPR, RPL = C::RPL, NL = C::NL, RR = C::RR, NW = 4;
+    __shared__ __align__(16) float wacc[NW][HG][D];
+    __shared__ float wm[NW][HG], wl[NW][HG];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rl = lane / LPR, dl = lane % LPR;
+    const int h0 = blockIdx.y * HG, g = h0 / rep, chunk = blockIdx.x, nch = gridDim.x;
+    const int8_t* kh = kc + (size_t)g * head_stride * C::EB;
+    const int8_t* vh = vc + (size_t)g * head_stride * C::EB;
+
+    struct Round {
+        uint4 k[NL], v[NL];
+        float ks[Q8 ? NL : 1], vs[Q8 ? NL : 1];
+    };
+    auto load = [&](Round& r, int base) {   // base < ctx
+        const int n = min(RR, ctx - base);
+        const auto kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(kh + (size_t)base * D * C::EB), 0, n * D * C::EB, 0x00020000);
+        const auto vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(vh + (size_t)base * D * C::EB), 0, n * D * C::EB, 0x00020000);
+#pragma unroll
+        for (int j = 0; j < NL; ++j)
+            r.k[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(kr, 16 * lane + 1024 * j, 0, 0));
+        if constexpr (Q8) {
+            const auto sr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(ks + base), 0, n * 4, 0x00020000);
+            const auto tr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vs + base), 0, n * 4, 0x00020000);
+#pragma unroll
+            for (int j = 0; j < NL; ++j) {
+                r.ks[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sr, 4 * (j * RPL + rl), 0, 0));
+                r.vs[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(tr, 4 * (j * RPL + rl), 0, 0));
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NL; ++j)
+            r.v[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(vr, 16 * lane + 1024 * j, 0, 0));
+    };
+
+    float qr[HG][EPL], acc[HG][EPL], m[HG], m2[HG], l[HG];
+#pragma unroll
+    for (int h = 0; h < HG; ++h) {
+#pragma unroll
+        for (int e = 0; e < EPL; e += 4) {
+            const float4 x = *reinterpret_cast<const float4*>(q + (size_t)(h0 + h) * D + dl * EPL + e);
+            qr[h][e] = qsign * x.x; qr[h][e + 1] = qsign * x.y; qr[h][e + 2] = qsign * x.z; qr[h][e + 3] = qsign * x.w;
+        }
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[h][e] = 0.f;
+        m[h] = kNegInf;
+        m2[h] = l[h] = 0.f;
+    }
+    auto compute = [&](const Round& r, int base) {
+        float s[NL][HG];
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+            float kf[EPL];
+            words_f32<KVT>(r.k[j], kf);
+#pragma unroll
+            for (int h = 0; h < HG; ++h) {
+                float a = 0.f;
+#pragma unroll
+                for (int e = 0; e < EPL; ++e) a = fmaf(qr[h][e], kf[e], a);
+                s[j][h] = row_sum<LPR>(a);
+                if constexpr (Q8) s[j][h] *= r.ks[j];
+            }
+        }
+        const bool tail = base + RR > ctx;
+        if (tail) {
+#pragma unroll
+            for (int j = 0; j < NL; ++j)
+#pragma unroll
+                for (int h = 0; h < HG; ++h) s[j][h] = base + j * RPL + rl < ctx ? s[j][h] : kNegInf;
+        }
+#pragma unroll
+        for (int h = 0; h < HG; ++h) {
+            float mt = s[0][h];
+#pragma unroll
+            for (int j = 1; j < NL; ++j) mt = fmaxf(mt, s[j][h]);
+            const float mn = fmaxf(m[h], across_rows<LPR, true>(mt));
+            const float m2n = mn == kNegInf ? 0.f : mn * sl2;
+            const float corr = m[h] == kNegInf ? 0.f : __builtin_amdgcn_exp2f(m2[h] - m2n);
+            m[h] = mn;
+            m2[h] = m2n;
+            l[h] *= corr;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) acc[h][e] *= corr;
+#pragma unroll
+            for (int j = 0; j < NL; ++j) {
+                float p = __builtin_amdgcn_exp2f(fmaf(s[j][h], sl2, -m2n));
+                if (tail) p = base + j * RPL + rl < ctx ? p : 0.f;
+                l[h] += p;
+                s[j][h] = Q8 ? p * r.vs[j] : p;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+            float vf[EPL];
+            words_f32<KVT>(r.v[j], vf);
+#pragma unroll
+            for (int h = 0; h < HG; ++h)
+#pragma unroll
+                for (int e = 0; e < EPL; ++e) acc[h][e] = fmaf(s[j][h], vf[e], acc[h][e]);
+        }
+    };
+
+    // The wave's rounds: w, w + 4, ... of the chunk's 4 * rounds, while they begin inside the context.
+    const int c0 = chunk * NW * rounds * RR + w * RR;
+    const int left = ctx - c0, mine = left <= 0 ? 0 : min(rounds, (left + NW * RR - 1) / (NW * RR));
+    if (mine > 0) {
+        Round r0, r1;
+        load(r0, c0);
+        for (int i = 0; i < mine; i += 2) {
+            const int base = c0 + i * NW * RR;
+            if (i + 1 < mine) load(r1, base + NW * RR);
+            compute(r0, base);
+            if (i + 1 < mine) {
+                if (i + 2 < mine) load(r0, base + 2 * NW * RR);
+                compute(r1, base + NW * RR);
+            }
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < HG; ++h) {
+        const float lw = across_rows<LPR, false>(l[h]);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[h][e] = across_rows_dims<LPR>(acc[h][e]);
+        if (rl == 0) {
+#pragma unroll
+            for (int e = 0; e < EPL; e += 4)
+                *reinterpret_cast<float4*>(&wacc[w][h][dl * EPL + e]) =
+                    make_float4(acc[h][e], acc[h][e + 1], acc[h][e + 2], acc[h][e + 3]);
+        }
+        if (lane == 0) {
+            wm[w][h] = m[h] == kNegInf ? kNegInf : m2[h];
+            wl[w][h] = lw;
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < HG * D; i += 256) {
+        const int h = i / D, dd = i % D;
+        float M = wm[0][h], L = 0.f, x = 0.f;
+#pragma unroll
+        for (int k = 1; k < NW; ++k) M = fmaxf(M, wm[k][h]);
+#pragma unroll
+        for (int k = 0; k < NW; ++k) {
+            const float f = wm[k][h] == kNegInf ? 0.f : __builtin_amdgcn_exp2f(wm[k][h] - M);
+            L += f * wl[k][h];
+            x += f * wacc[k][h][dd];
+        }
+        if (nch == 1) {
+            out[(size_t)(h0 + h) * D + dd] = L > 0.f ? x * (1.f / L) : 0.f;
+        } else {
+            float* p = part + ((size_t)(h0 + h) * nch + chunk) * (D + 2);
+            p[dd] = x;
+            if (dd == 0) {
+                p[D] = M;
+                p[D + 1] = L;
+            }
+        }
+    }
+}
+
+// out = sum_c 2^(m_c - M) acc_c / sum_c 2^(m_c - M) l_c over a head's chunks.
+// Thread (group gi, dim d) takes chunks gi, gi + G, ... in passes of B whose loads
+// are all issued before any is used; the groups merge through LDS.
+template <int D>
+__global__ __launch_bounds__(512) void attn_decode_merge_kernel(const float* __restrict__ part, int nch,
+                                                                float* __restrict__ out) {
+    constexpr int G = 512 / D, B = 16;
+    __shared__ float sm[G][D], sl[G][D], so[G][D];
+    const int h = blockIdx.x, gi = threadIdx.x / D, d = threadIdx.x % D;
+    const float* p = part + (size_t)h * nch * (D + 2);
+    float M = kNegInf, L = 0.f, o = 0.f;
+    for (int c0 = gi; c0 < nch; c0 += G * B) {
+        float pm[B], pl[B], po[B], mb = M;
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const float* pc = p + (size_t)min(c0 + b * G, nch - 1) * (D + 2);
+            pm[b] = pc[D];
+            pl[b] = pc[D + 1];
+            po[b] = pc[d];
+        }
+#pragma unroll
+        for (int b = 0; b < B; ++b) mb = fmaxf(mb, pm[b]);   // a repeated last chunk does no harm
+        const float f = M == kNegInf ? 0.f : __builtin_amdgcn_exp2f(M - mb);
+        L *= f;
+        o *= f;
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const float e = c0 + b * G < nch && pm[b] != kNegInf ? __builtin_amdgcn_exp2f(pm[b] - mb) : 0.f;
+            L += e == 0.f ? 0.f : e * pl[b];
+            o += e == 0.f ? 0.f : e * po[b];
+        }
+        M = mb;
+    }
+    sm[gi][d] = M;
+    sl[gi][d] = L;
+    so[gi][d] = o;
+    __syncthreads();
+    if (gi) return;
+    float Mt = sm[0][d], Lt = 0.f, ot = 0.f;
+#pragma unroll
+    for (int k = 1; k < G; ++k) Mt = fmaxf(Mt, sm[k][d]);
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+        const float f = sm[k][d] == kNegInf ? 0.f : __builtin_amdgcn_exp2f(sm[k][d] - Mt);
+        Lt += f * sl[k][d];
+        ot += f * so[k][d];
+    }
+    out[(size_t)h * D + d] = Lt > 0.f ? ot * (1.f / Lt) : 0.f;
+}
+
 // ---- stand-alone decode attention in one launch ----------------------------------
 // vlrf_hip_attn_decode / attn_f32 at T = 1 (AttentionBlock::flash_attn_head for
 // one query row over the cache, attention.hpp:207-309, non-causal): workgroup
@@ -1350,8 +1640,8 @@ int launch_attn_decode(hipStream_t s, const float* q, const void* kc, const void
                "attn_decode: chunked form for %d chunks does not apply", fz.nch);
         const dim3 cgrid(8 * rep * ((n_kv * fz.nch + 7) / 8));
 #define VH_CHK(KT, R)                                                                                         \
-    VH_LAUNCH((attn_decode_single_kernel<KT, R, true, kCH>), cgrid, dim3(kCH), 0, s, q, k8, v8, ks, vs,       \
-                       head_stride, ctx_len, ctx_dev, scale, fz.chunks, fz, fz.nch)
+    VH_LAUNCH((attn_decode_single_kernel<KT, R, kCH>), cgrid, dim3(kCH), 0, s, q, k8, v8, ks, vs,       \
+                       head_stride, ctx_dev, scale, fz.chunks, fz, fz.nch)
 #define VH_CHK_R(KT)                     \
     switch (rep) {                       \
         case 1: VH_CHK(KT, 1); break;    \
@@ -1370,11 +1660,68 @@ int launch_attn_decode(hipStream_t s, const float* q, const void* kc, const void
         return VLRF_HIP_OK;
     }
     static const bool chunks_on = [] {
-        const char* e = std::getenv("VLRF_HIP_ATTN_CHUNKS");   // "0": the split-K pair of launches instead
+        const char* e = std::getenv("VLRF_HIP_ATTN_CHUNKS");   // "0": the rows kernel and its merge instead
         return !(e && e[0] == '0');
     }();
-    if (chunks_on && !fuse && ctr && !ctx_dev && d_head == 64 && ctx_len <= kChunksMaxCtx &&
-        n_heads <= kSmallMaxTiles) {
+    // The one-launch chunked form reads K/V once per query head and is bound by
+    // its latency; from 8 MiB of K/V the rows kernel, which reads them once per
+    // four heads, is faster although it merges in a launch of its own.  us, chunked /
+    // rows, d 64: 32/4 heads, Q8_0 4096 keys (2.1 MB) 8.5 / 9.7; 16/8, f32 1126 (4.6)
+    // 6.7 / 7.3; 8/8, Q8_0 8000 (8.2) 9.0 / 8.1; 32/4, f32 8000 (16) 20.9 / 12.1.
+    const size_t kv_bytes = 2 * (size_t)ctx_len * n_kv * d_head * kv_elem_bytes(kv_dtype);
+    const bool chunked = chunks_on && !fuse && ctr && d_head == 64 && ctx_len <= kChunksMaxCtx &&
+                         n_heads <= kSmallMaxTiles && kv_bytes < (8u << 20);
+    if (!fuse && !chunked) {
+        // Workgroups of four waves, a round of 8 KiB of K per wave (rr8 rows), as
+        // many rounds as leave about one workgroup per CU (it holds 300 registers a
+        // lane: 512 ran 25.9 against 22.2 us at 15001 keys, 8 KV heads, d 128, f16).
+        // Fewer workgroups than CUs: rounds of a quarter of that, so four times as
+        // many (32/8 heads, d 128, Q8_0 4096: 13.3 -> 12.2 us; 8/2 heads, 582: 11.6 ->
+        // 9.3), unless one chunk holds all the keys and needs no merge.
+        // Before: 64-key workgroups and a serial merge of their partials, 56.3 us
+        // at 15001 keys f16 (100.2 f32, 44.5 Q8_0), now 22.3 (28.5, 20.8).
+        VH_ARG(!ctx_dev, "attn_decode: a device position needs the fused form");
+        const float sl2 = (float)(std::fabs((double)scale) * 1.4426950408889634), qsign = scale < 0.f ? -1.f : 1.f;
+        const int hg = rep < 4 ? rep : 4, groups = n_heads / hg;
+        const int rr8 = 8 * 1024 / (d_head * kv_elem_bytes(kv_dtype));
+        const int wg8 = (ctx_len + 4 * rr8 - 1) / (4 * rr8);
+        const bool big = wg8 == 1 || (long)wg8 * groups >= 256;
+        const int rows = big ? 4 * rr8 : rr8;   // of a workgroup's round
+        int rounds = (int)(((long)((ctx_len + rows - 1) / rows) * groups + 255) / 256);
+        rounds = rounds > (64 + rows - 1) / rows ? rounds : (64 + rows - 1) / rows;   // at most n_splits chunks
+        const int nch = (ctx_len + rows * rounds - 1) / (rows * rounds);
+#define VH_RW(D, HG, KT)                                                                                           \
+    if (big)                                                                                                       \
+        VH_LAUNCH((attn_decode_rows_kernel<D, HG, KT, 8>), dim3(nch, groups), dim3(256), 0, s, q, k8, v8, ks, vs,  \
+                  head_stride, ctx_len, rep, rounds, sl2, qsign, part, out);                                       \
+    else                                                                                                           \
+        VH_LAUNCH((attn_decode_rows_kernel<D, HG, KT, 2>), dim3(nch, groups), dim3(256), 0, s, q, k8, v8, ks, vs,  \
+                  head_stride, ctx_len, rep, rounds, sl2, qsign, part, out)
+#define VH_RW_H(D, KT)                 \
+    switch (hg) {                      \
+        case 1: VH_RW(D, 1, KT); break; \
+        case 2: VH_RW(D, 2, KT); break; \
+        default: VH_RW(D, 4, KT); break; \
+    }
+#define VH_RW_T(D)                                                  \
+    switch (kv_dtype) {                                             \
+        case VLRF_HIP_KV_Q8_0: VH_RW_H(D, VLRF_HIP_KV_Q8_0) break;  \
+        case VLRF_HIP_KV_F16: VH_RW_H(D, VLRF_HIP_KV_F16) break;    \
+        default: VH_RW_H(D, VLRF_HIP_KV_F32) break;                 \
+    }
+        if (d_head == 64) { VH_RW_T(64) } else { VH_RW_T(128) }
+#undef VH_RW_T
+#undef VH_RW_H
+#undef VH_RW
+        VH_LAUNCHED();
+        if (nch > 1) {
+            if (d_head == 64) VH_LAUNCH((attn_decode_merge_kernel<64>), dim3(n_heads), dim3(512), 0, s, part, nch, out);
+            else VH_LAUNCH((attn_decode_merge_kernel<128>), dim3(n_heads), dim3(512), 0, s, part, nch, out);
+            VH_LAUNCHED();
+        }
+        return VLRF_HIP_OK;
+    }
+    if (chunked) {
         // One launch: the smallest chunk (64..512 rows) that splits the context
         // into at most kAttnMaxChunks chunks; nch <= ceil(ctx_len / 64) = n_splits,
         // so the partials fit the split-K buffer.
@@ -1410,25 +1757,24 @@ int launch_attn_decode(hipStream_t s, const float* q, const void* kc, const void
         VH_LAUNCHED();
         return VLRF_HIP_OK;
     }
-    if (d_head == 64 && head_stride / d_head <= kSPMaxCtx && (!fuse || n_kv <= 8)) {
-#define VH_SP(KT, R, FU)                                                                                     \
-    VH_LAUNCH((attn_decode_single_kernel<KT, R, FU>), dim3(n_heads), dim3(64 * kSPWaves), 0, s, q, k8,       \
-                       v8, ks, vs, head_stride, ctx_len, ctx_dev, scale, out, fz, 0)
-#define VH_SP_R(KT, FU)                       \
+    if (d_head == 64 && head_stride / d_head <= kSPMaxCtx && n_kv <= 8) {
+#define VH_SP(KT, R)                                                                                         \
+    VH_LAUNCH((attn_decode_single_kernel<KT, R>), dim3(n_heads), dim3(64 * kSPWaves), 0, s, q, k8,       \
+                       v8, ks, vs, head_stride, ctx_dev, scale, out, fz, 0)
+#define VH_SP_R(KT)                       \
     switch (rep) {                            \
-        case 1: VH_SP(KT, 1, FU); break;      \
-        case 2: VH_SP(KT, 2, FU); break;      \
-        case 4: VH_SP(KT, 4, FU); break;      \
-        default: VH_SP(KT, 8, FU); break;     \
+        case 1: VH_SP(KT, 1); break;      \
+        case 2: VH_SP(KT, 2); break;      \
+        case 4: VH_SP(KT, 4); break;      \
+        default: VH_SP(KT, 8); break;     \
     }
-#define VH_SP_T(FU)                                                 \
+#define VH_SP_T()                                                 \
     switch (kv_dtype) {                                             \
-        case VLRF_HIP_KV_Q8_0: VH_SP_R(VLRF_HIP_KV_Q8_0, FU) break; \
-        case VLRF_HIP_KV_F16: VH_SP_R(VLRF_HIP_KV_F16, FU) break;   \
-        default: VH_SP_R(VLRF_HIP_KV_F32, FU) break;                \
+        case VLRF_HIP_KV_Q8_0: VH_SP_R(VLRF_HIP_KV_Q8_0) break; \
+        case VLRF_HIP_KV_F16: VH_SP_R(VLRF_HIP_KV_F16) break;   \
+        default: VH_SP_R(VLRF_HIP_KV_F32) break;                \
     }
-        if (fuse) { VH_SP_T(true) }
-        else { VH_SP_T(false) }
+        VH_SP_T()
 #undef VH_SP_T
 #undef VH_SP_R
 #undef VH_SP
@@ -1436,29 +1782,23 @@ int launch_attn_decode(hipStream_t s, const float* q, const void* kc, const void
         return VLRF_HIP_OK;
     }
     dim3 grid(n_splits, n_kv), block(kAttnThreads);
-#define VH_AD(D, R, T, FU)                                                                          \
-    VH_LAUNCH((attn_decode_partial_kernel<D, R, T, FU>), grid, block, 0, s, q, k8, v8, ks,          \
-                       vs, head_stride, ctx_len, ctx_dev, n_splits, scale, part, fz)
-#define VH_AD_R(D, T, FU)                       \
+#define VH_AD(D, R, T)                                                                          \
+    VH_LAUNCH((attn_decode_partial_kernel<D, R, T>), grid, block, 0, s, q, k8, v8, ks,          \
+                       vs, head_stride, ctx_dev, n_splits, scale, part, fz)
+#define VH_AD_R(D, T)                       \
     switch (rep) {                              \
-        case 1: VH_AD(D, 1, T, FU); break;      \
-        case 2: VH_AD(D, 2, T, FU); break;      \
-        case 4: VH_AD(D, 4, T, FU); break;      \
-        default: VH_AD(D, 8, T, FU); break;     \
+        case 1: VH_AD(D, 1, T); break;      \
+        case 2: VH_AD(D, 2, T); break;      \
+        case 4: VH_AD(D, 4, T); break;      \
+        default: VH_AD(D, 8, T); break;     \
     }
-#define VH_AD_T(D, FU)                                                   \
+#define VH_AD_T(D)                                                   \
     switch (kv_dtype) {                                                  \
-        case VLRF_HIP_KV_Q8_0: VH_AD_R(D, VLRF_HIP_KV_Q8_0, FU) break;   \
-        case VLRF_HIP_KV_F16: VH_AD_R(D, VLRF_HIP_KV_F16, FU) break;     \
-        default: VH_AD_R(D, VLRF_HIP_KV_F32, FU) break;                  \
+        case VLRF_HIP_KV_Q8_0: VH_AD_R(D, VLRF_HIP_KV_Q8_0) break;   \
+        case VLRF_HIP_KV_F16: VH_AD_R(D, VLRF_HIP_KV_F16) break;     \
+        default: VH_AD_R(D, VLRF_HIP_KV_F32) break;                  \
     }
-    if (d_head == 64) {
-        if (fuse) { VH_AD_T(64, true) }
-        else { VH_AD_T(64, false) }
-    } else {
-        if (fuse) { VH_AD_T(128, true) }
-        else { VH_AD_T(128, false) }
-    }
+    if (d_head == 64) { VH_AD_T(64) } else { VH_AD_T(128) }
 #undef VH_AD_T
 #undef VH_AD_R
 #undef VH_AD
