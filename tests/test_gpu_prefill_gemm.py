@@ -148,6 +148,60 @@ def test_split_k_swiglu_mid_m(ctx, orc, monkeypatch, dtype, M, Fd, K):
     assert rel_err(got, unsplit) <= 2e-5, rel_err(got, unsplit)
 
 
+def _bf16(x):
+    """x rounded to bf16 (nearest even)."""
+    u = np.ascontiguousarray(x, np.float32).view(np.uint32)
+    return ((u + 0x7FFF + ((u >> 16) & 1)) & np.uint32(0xFFFF0000)).view(np.float32)
+
+
+@pytest.mark.parametrize("dtype", [V.DT_Q8_0, V.DT_Q4_0])
+@pytest.mark.parametrize("M,N,K,res", [(17, 300, 64, False), (64, 37, 576, True), (65, 700, 1216, False),
+                                       (128, 520, 5504, True), (100, 129, 8128, False),       # 17..128 rows
+                                       (129, 100, 64, True), (130, 300, 704, False), (300, 515, 5504, True),
+                                       (257, 130, 8128, False), (600, 260, 1984, True)])      # more
+def test_gemm_uneven_k_slices(ctx, monkeypatch, dtype, M, N, K, res):
+    """K of any number of 64-column steps: odd step counts, slices that do not
+    divide them (a shorter last one), one-step slices.  bf16 products summed
+    over K in any order in f32 are within (K + slices) eps of their absolute sum of each other:
+    the forms agree as _check_forms says, and with 64-bit sums of the same bf16 operands."""
+    print(f"[case] uneven K slices dtype={dtype} M={M} N={N} K={K} res={res}", flush=True)
+    x = F.normal(28, f"ux{M}x{K}", M * K).reshape(M, K)
+    r = F.normal(28, f"ur{M}x{N}", M * N).reshape(M, N)
+    dx = ctx.to_device(x)
+    dec = []
+
+    def run():
+        w, d = _weight(ctx, 28, f"U{N}x{K}", N, K, dtype)
+        dec.append(d)
+        dy = ctx.to_device(r) if res else ctx.alloc(M * N * 4)
+        ctx.qlinear(w, dx, dy, M, residual=dy if res else None)
+        return dy.download((M, N))
+
+    a, b, c = _all_forms(monkeypatch, run)
+    _check_forms(a, b, c)
+    xb, wb = (_bf16(t).astype(np.float64) for t in (x, dec[0]))
+    ref = xb @ wb.T + (r if res else 0)
+    bound = (K + 40) * 2.0 ** -24 * (np.abs(xb) @ np.abs(wb).T + (np.abs(r) if res else 0))
+    assert (np.abs(a - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("M,Fd,K", [(33, 200, 704), (90, 515, 1984), (300, 130, 5504)])
+def test_swiglu_uneven_k_slices(ctx, monkeypatch, M, Fd, K):
+    print(f"[case] uneven K slices swiglu M={M} F={Fd} K={K}", flush=True)
+    x = F.normal(29, f"vx{M}x{K}", M * K).reshape(M, K)
+    dx = ctx.to_device(x)
+
+    def run():
+        wg, _ = _weight(ctx, 29, f"VG{Fd}x{K}", Fd, K, V.DT_Q4_0)
+        wu, _ = _weight(ctx, 29, f"VU{Fd}x{K}", Fd, K, V.DT_Q4_0)
+        dh = ctx.alloc(M * Fd * 4)
+        ctx.qlinear_swiglu(wg, wu, dx, dh, M)
+        return dh.download((M, Fd))
+
+    a, b, c = _all_forms(monkeypatch, run)
+    _check_forms(a, b, c)
+
+
 def _check_forms(a, b, c):
     """Expansion and in-LDS forms identical bit for bit; the in-register form
     identical too, except where the GEMM's few tiles make the two others

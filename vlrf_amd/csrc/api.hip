@@ -606,6 +606,23 @@ size_t vlrf_hip_weight_bytes(vlrf_hip_weight_t w) {
     return weight_device_bytes(w->w.dtype, w->w.N, w->w.K) + (w->w.bf ? (size_t)w->w.N * w->w.K * 2 : 0);
 }
 
+}  // extern "C"
+
+// Scratch of a GEMM of M > 16 rows: the bf16 rows, then the K-split partial sums;
+// where both together cannot be had, the rows alone (K then stays whole).
+static int gemm_scratch(Ctx* ctx, size_t a_bytes, size_t p_bytes, float** a, float** part) {
+    *part = nullptr;
+    int rc = ctx->scratch(a_bytes + p_bytes, a);
+    if (!rc) {
+        if (p_bytes) *part = reinterpret_cast<float*>(reinterpret_cast<char*>(*a) + a_bytes);
+        return VLRF_HIP_OK;
+    }
+    (void)hipGetLastError();
+    return p_bytes ? ctx->scratch(a_bytes, a) : rc;
+}
+
+extern "C" {
+
 // M <= 16 runs the f32 GEMV / small-M kernels; larger M (prefill) runs the
 // MFMA GEMM on bf16 operands (x, optionally RMS-normalised, is rounded to bf16
 // in the context's scratch buffer first).
@@ -623,14 +640,12 @@ int vlrf_hip_qlinear(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t w, const float* x, fl
     }
     if (M <= 16) return launch_qlinear(ctx->stream, w->w, x, y, M, norm_w, eps, residual);
     VH_ARG(x && y, "qlinear: null activation pointer");
-    // Scratch: the bf16 rows, then the K-split partial sums (17 <= M <= 128).
     const size_t a_bytes = ((size_t)M * w->w.K * sizeof(uint16_t) + 255) & ~(size_t)255;
     const size_t p_bytes = qgemm_part_bytes(w->w, M, false);
-    float* scratch = nullptr;
-    int rc = ctx->scratch(a_bytes + p_bytes, &scratch);
+    float *scratch = nullptr, *part = nullptr;
+    int rc = gemm_scratch(ctx, a_bytes, p_bytes, &scratch, &part);
     if (rc) return rc;
     uint16_t* a = reinterpret_cast<uint16_t*>(scratch);
-    float* part = p_bytes ? reinterpret_cast<float*>(reinterpret_cast<char*>(scratch) + a_bytes) : nullptr;
     rc = launch_rows_to_bf16(ctx->stream, x, norm_w, a, M, w->w.K, eps);
     if (rc) return rc;
     return launch_qgemm(ctx->stream, w->w, a, M, residual, y, part);
@@ -652,11 +667,10 @@ int vlrf_hip_qlinear_swiglu(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t wg, vlrf_hip_w
     VH_ARG(x && h, "swiglu: null activation pointer");
     const size_t a_bytes = ((size_t)M * wg->w.K * sizeof(uint16_t) + 255) & ~(size_t)255;
     const size_t p_bytes = qgemm_part_bytes(wg->w, M, true);
-    float* scratch = nullptr;
-    int rc = ctx->scratch(a_bytes + p_bytes, &scratch);
+    float *scratch = nullptr, *part = nullptr;
+    int rc = gemm_scratch(ctx, a_bytes, p_bytes, &scratch, &part);
     if (rc) return rc;
     uint16_t* a = reinterpret_cast<uint16_t*>(scratch);
-    float* part = p_bytes ? reinterpret_cast<float*>(reinterpret_cast<char*>(scratch) + a_bytes) : nullptr;
     rc = launch_rows_to_bf16(ctx->stream, x, norm_w, a, M, wg->w.K, eps);
     if (rc) return rc;
     return launch_qgemm_swiglu(ctx->stream, wg->w, wu->w, a, M, h, false, part);

@@ -560,7 +560,7 @@ __global__ __launch_bounds__(T::NT) void mfma_bgemm_kernel(
     const int wm = wave / T::WC, wn = wave % T::WC;
     const int m0 = blockIdx.y * T::BM;
     const int n0 = blockIdx.x * (SWIGLU ? BN / 2 : BN);   // first output column
-    const int k0 = blockIdx.z * kl;                        // this launch's K range: k0 .. k0 + kl (rows K long)
+    const int k0 = blockIdx.z * kl;                        // this slice's K range: k0 .. min(k0 + kl, K) (rows K long)
 
     // Sources of K step 0 (step k adds RB bytes) and destinations: wave w's
     // load `it` fills rows RPL (NW it + w) .. + RPL - 1 of the tile, lane l row
@@ -682,7 +682,7 @@ __global__ __launch_bounds__(T::NT) void mfma_bgemm_kernel(
     constexpr int W_ALL = 0x70;                                                           // vmcnt(0) lgkmcnt(0)
     constexpr int W_IN = ((NS - 2) * LPS & 15) | (7 << 4) | (((NS - 2) * LPS >> 4) << 14);   // vmcnt((NS-2) LPS) lgkmcnt(0)
     constexpr int W_PRO = ((NS - 1) * LPS & 15) | (7 << 4) | (15 << 8) | (((NS - 1) * LPS >> 4) << 14);
-    const int nk = kl / T::BK;
+    const int nk = min(kl, K - k0) / T::BK;
 #pragma unroll
     for (int j = 0; j < NS; ++j) load(min(j, nk - 1), j);
     __builtin_amdgcn_s_waitcnt(W_PRO);   // step 0's loads in: the newer NS - 1 stages pending
@@ -860,7 +860,7 @@ __global__ __launch_bounds__(T::NT) void mfma_dqgemm_kernel(
     const int wm = wave / T::WC, wn = wave % T::WC;
     const int m0 = blockIdx.y * T::BM;
     const int n0 = blockIdx.x * (SWIGLU ? BN / 2 : BN);   // first output column
-    const int k0 = blockIdx.z * kl;                        // this launch's K range: k0 .. k0 + kl (rows K long)
+    const int k0 = blockIdx.z * kl;                        // this slice's K range: k0 .. min(k0 + kl, K) (rows K long)
 
     const char* ga[T::A_IT];
 #pragma unroll
@@ -1012,7 +1012,7 @@ __global__ __launch_bounds__(T::NT) void mfma_dqgemm_kernel(
     // Prologue, so that every step finds the same loads in flight: codes 0
     // (decoded into W buffer 0), then A 0 .. NSA - 3, and the pairs (A
     // NSA - 2, codes 1), (A NSA - 1, codes 2).
-    const int nk = kl / T::BK;
+    const int nk = min(kl, K - k0) / T::BK;
     load_w(0, cq0);
     cq0.template wait<0>();
     store_w(cq0, 0, 0, NC);
@@ -1045,10 +1045,11 @@ __global__ __launch_bounds__(T::NT) void mfma_dqgemm_kernel(
         phase_refill(fa[1], fb[1], sn, s1, fa[0], fb[0], min(k + NSA, nk - 1), st, min(k + 3, nk - 1), qn);
         st = sn;
     };
-    for (int k = 0; k < nk; k += 2) {
+    for (int k = 0; k + 1 < nk; k += 2) {
         step(k, cq1);
         step(k + 1, cq0);
     }
+    if (nk & 1) step(nk - 1, cq1);
     cq0.template wait<0>();   // nothing outlives the workgroup
     cq1.template wait<0>();
 
@@ -1295,10 +1296,10 @@ void launch_dqgemm(hipStream_t s, const uint16_t* a, const DevWeight& w0, const 
                            M, nn, w0.K, w0.K, w0.N, res, o);
 }
 
-// Q8_0 / Q4_0 weights with K a multiple of 128 (whole 64-element K-step pairs).
+// Q8_0 / Q4_0 weights with K a multiple of 64 (whole K steps).
 bool dqgemm_supported(const DevWeight& w) {
     const char* e = getenv("VLRF_HIP_PREFILL_DQ");   // "0": the in-register decode instead
-    return !(e && e[0] == '0') && (w.dtype == VLRF_HIP_DT_Q8_0 || w.dtype == VLRF_HIP_DT_Q4_0) && w.K % 128 == 0;
+    return !(e && e[0] == '0') && (w.dtype == VLRF_HIP_DT_Q8_0 || w.dtype == VLRF_HIP_DT_Q4_0) && w.K % 64 == 0;
 }
 
 // The tile plan of launch_bgemm_plan_t over codes, with half tiles of half
@@ -1334,8 +1335,8 @@ void launch_dqgemm_plan(hipStream_t s, const uint16_t* a, const DevWeight& w0, c
 // split into S contiguous slices instead, each slice's f32 sums written to a
 // partial buffer ([S][M][N], SwiGLU [S][M][2N]: gate, then up), and
 // splitk_reduce_kernel adds the slices in order (the same sum on every run)
-// and applies the epilogue.  S is the largest divisor of K / 128 whose
-// workgroups fit one round of the CUs and whose slices keep at least 8 K
+// and applies the epilogue.  S is the most slices whose
+// workgroups fit one round of the CUs and which keep at least 8 K
 // steps (the pipeline's prologue and the partial stores are per slice; 8B
 // QKV at M = 128, 48 column tiles: 4 slices 26.8 us, 8 slices 1.5 rounds
 // 30.2 us).  Measured while S was the smallest divisor reaching a round:
@@ -1421,49 +1422,65 @@ void launch_splitk_reduce(hipStream_t s, const float* part, int S, int M, int N,
 using SplitTile64 = BTile<64, 256, 2, 4>;     // M <= 64: 8 waves of 32 x 64
 using SplitTile128 = BTile<128, 128, 4, 2>;   // 65 <= M <= 128: 8 waves of 32 x 64
 
-int splitk_slices(const DevWeight& w, int M, bool swiglu, int cus) {
-    const int bn = M <= 64 ? SplitTile64::BN : SplitTile128::BN;
-    const long nt = (w.N + (swiglu ? bn / 2 : bn) - 1) / (swiglu ? bn / 2 : bn);
-    const int kb = w.K / 128;
-    constexpr int kMinSteps = 8;   // K steps per slice at least (2 and 4 measured slower in sum)
-    int S = 1;
-    for (int d = 1; d <= kb; ++d) {
-        if (kb % d) continue;
-        if (w.K / 64 / d < kMinSteps || (d > 1 && nt * d > cus)) break;
-        S = d;
-    }
-    return S;
+// A split of K's steps of 64: S slices of kl columns, the last one with what is left.
+struct KSplit {
+    int S, kl;
+};
+
+// As many slices as fit one round of the CUs beside each other (tiles output
+// tiles), of at least 8 steps: a number down to 3/4 of that which divides the
+// steps, if there is one (8B QKV at M = 100, 48 tiles of 64 steps: 4 slices 23.9
+// us, 5 uneven ones 24.4), else that many, as even as whole steps allow.  (us at
+// Q8_0, slices that had to divide K / 128 or none -> these: 4123 x 10944, M = 105,
+// 221 -> 33.5; 2048 x 5504, M = 128, 60 -> 22; 4757 x 9856, M = 395, 122 -> 79;
+// 773 x 10432, M = 20, 191 -> 21.6.)
+KSplit split_k(long tiles, int K, int cus) {
+    const int steps = K / 64;
+    long S = cus / tiles < steps / 8 ? cus / tiles : steps / 8;
+    if (S < 1) S = 1;
+    for (long d = S; 4 * d >= 3 * S; --d)
+        if (steps % d == 0) {
+            S = d;
+            break;
+        }
+    const int per = (int)((steps + S - 1) / S);
+    return {(steps + per - 1) / per, per * 64};
+}
+
+KSplit mid_split(const DevWeight& w, int M, bool swiglu, int cus) {
+    const int bn = (M <= 64 ? SplitTile64::BN : SplitTile128::BN) / (swiglu ? 2 : 1);
+    return split_k((w.N + bn - 1) / bn, w.K, cus);
 }
 
 template <class T, int WT, int EPI>
-void launch_dq_split_t(hipStream_t s, const uint16_t* a, const DevWeight& w0, const DevWeight* w1, int M, int S,
+void launch_dq_split_t(hipStream_t s, const uint16_t* a, const DevWeight& w0, const DevWeight* w1, int M, KSplit ks,
                        const float* residual, void* out, float* part) {
     constexpr bool SW = EPI >= 2;
     constexpr int TN = SW ? T::BN / 2 : T::BN;
     const int N = w0.N, K = w0.K;
-    const dim3 grid((N + TN - 1) / TN, (M + T::BM - 1) / T::BM, S);
+    const dim3 grid((N + TN - 1) / TN, (M + T::BM - 1) / T::BM, ks.S);
     const uint8_t* qb = SW ? w1->q : w0.q;
     const __half* db = SW ? w1->d : w0.d;
-    if (S == 1) {
+    if (ks.S == 1) {
         hipLaunchKernelGGL((mfma_dqgemm_kernel<T, WT, EPI, 2>), grid, dim3(T::NT), 0, s, a, w0.q, w0.d, qb, db, M, N,
                            K, K, N, residual, out);
         return;
     }
     const int ldp = SW ? 2 * N : N;
     hipLaunchKernelGGL((mfma_dqgemm_kernel<T, WT, SW ? 7 : 6, 2>), grid, dim3(T::NT), 0, s, a, w0.q, w0.d, qb, db, M,
-                       N, K, K / S, ldp, nullptr, part);
-    launch_splitk_reduce<EPI>(s, part, S, M, N, ldp, residual, out);
+                       N, K, ks.kl, ldp, nullptr, part);
+    launch_splitk_reduce<EPI>(s, part, ks.S, M, N, ldp, residual, out);
 }
 
 template <int EPI>
-void launch_dq_split(hipStream_t s, const uint16_t* a, const DevWeight& w0, const DevWeight* w1, int M, int S,
+void launch_dq_split(hipStream_t s, const uint16_t* a, const DevWeight& w0, const DevWeight* w1, int M, KSplit ks,
                      const float* residual, void* out, float* part) {
     if (w0.dtype == VLRF_HIP_DT_Q8_0) {
-        if (M <= 64) launch_dq_split_t<SplitTile64, VLRF_HIP_DT_Q8_0, EPI>(s, a, w0, w1, M, S, residual, out, part);
-        else launch_dq_split_t<SplitTile128, VLRF_HIP_DT_Q8_0, EPI>(s, a, w0, w1, M, S, residual, out, part);
+        if (M <= 64) launch_dq_split_t<SplitTile64, VLRF_HIP_DT_Q8_0, EPI>(s, a, w0, w1, M, ks, residual, out, part);
+        else launch_dq_split_t<SplitTile128, VLRF_HIP_DT_Q8_0, EPI>(s, a, w0, w1, M, ks, residual, out, part);
     } else {
-        if (M <= 64) launch_dq_split_t<SplitTile64, VLRF_HIP_DT_Q4_0, EPI>(s, a, w0, w1, M, S, residual, out, part);
-        else launch_dq_split_t<SplitTile128, VLRF_HIP_DT_Q4_0, EPI>(s, a, w0, w1, M, S, residual, out, part);
+        if (M <= 64) launch_dq_split_t<SplitTile64, VLRF_HIP_DT_Q4_0, EPI>(s, a, w0, w1, M, ks, residual, out, part);
+        else launch_dq_split_t<SplitTile128, VLRF_HIP_DT_Q4_0, EPI>(s, a, w0, w1, M, ks, residual, out, part);
     }
 }
 
@@ -1471,49 +1488,42 @@ void launch_dq_split(hipStream_t s, const uint16_t* a, const DevWeight& w0, cons
 // The plans above fill the GPU at the 8B shapes only from about T = 2048: at
 // M = 256 the O and down GEMMs have 32 tiles.  Below a round of 256-row
 // x 128-column output tiles, both forms (over the bf16 expansions and over
-// the codes) split K into the same S slices -- the largest divisor of K / 128
-// whose workgroups still fit one round, slices of at least 8 K steps -- with
+// the codes) split K into the same slices -- as many as still fit one round, of
+// at least 8 K steps (split_k) -- with
 // the partial buffer and splitk_reduce_kernel of the 17..128-row path, so
 // the two forms still multiply and add the same numbers in the same order.
 // (8B layer, same box: against aiming at 3/4 of a round from below half a
 // round, T = 1024 0.677 -> 0.600 ms, its O and down now split in two; T =
 // 256 .. 768 within noise.  Aiming at a full round: T = 256 0.291 ms.)
-int big_split_slices(int M, int N, int K, int cus) {
+KSplit big_split(int M, int N, int K, int cus) {
     const long g0 = (long)((M + 255) / 256) * ((N + 127) / 128);
     const char* e = getenv("VLRF_HIP_PREFILL_SPLIT");   // "0": the unsplit plans at every M > 128
-    if ((e && e[0] == '0') || K % 128 || g0 >= cus) return 1;
-    const int kb = K / 128;
-    int S = 1;
-    for (int d = 1; d <= kb; ++d) {
-        if (kb % d) continue;
-        if (K / 64 / d < 8 || g0 * d > cus) break;
-        S = d;
-    }
-    return S;
+    if ((e && e[0] == '0') || g0 >= cus) return {1, K};
+    return split_k(g0, K, cus);
 }
 
 template <class T, int EPI>
-void launch_bgemm_split_t(hipStream_t s, const uint16_t* a, const DevWeight& w0, const DevWeight* w1, int M, int S,
+void launch_bgemm_split_t(hipStream_t s, const uint16_t* a, const DevWeight& w0, const DevWeight* w1, int M, KSplit ks,
                           const float* residual, void* out, float* part) {
     constexpr bool SW = EPI >= 2;
     constexpr int TN = SW ? T::BN / 2 : T::BN;
     const int N = w0.N, K = w0.K, ldp = SW ? 2 * N : N;
-    const dim3 grid((N + TN - 1) / TN, (M + T::BM - 1) / T::BM, S);
+    const dim3 grid((N + TN - 1) / TN, (M + T::BM - 1) / T::BM, ks.S);
     hipLaunchKernelGGL((mfma_bgemm_kernel<T, SW ? 7 : 6>), grid, dim3(T::NT), 0, s, a, w0.bf, SW ? w1->bf : w0.bf, M,
-                       N, K, K / S, ldp, nullptr, part);
-    launch_splitk_reduce<EPI>(s, part, S, M, N, ldp, residual, out);
+                       N, K, ks.kl, ldp, nullptr, part);
+    launch_splitk_reduce<EPI>(s, part, ks.S, M, N, ldp, residual, out);
 }
 
 // bf16: over the expansions (of both matrices for SwiGLU); else over the codes.
 template <int EPI>
 void launch_big_split(hipStream_t s, bool bf16, const uint16_t* a, const DevWeight& w0, const DevWeight* w1, int M,
-                      int S, const float* residual, void* out, float* part) {
+                      KSplit ks, const float* residual, void* out, float* part) {
     using TP = BTile<256, 128, 4, 2>;   // plain: 256 x 128 tiles
     using TS = BTile<256, 256, 2, 4>;   // SwiGLU: 256 rows x 128 gate and 128 up rows
     using T = typename std::conditional<(EPI >= 2), TS, TP>::type;
-    if (bf16) launch_bgemm_split_t<T, EPI>(s, a, w0, w1, M, S, residual, out, part);
-    else if (w0.dtype == VLRF_HIP_DT_Q8_0) launch_dq_split_t<T, VLRF_HIP_DT_Q8_0, EPI>(s, a, w0, w1, M, S, residual, out, part);
-    else launch_dq_split_t<T, VLRF_HIP_DT_Q4_0, EPI>(s, a, w0, w1, M, S, residual, out, part);
+    if (bf16) launch_bgemm_split_t<T, EPI>(s, a, w0, w1, M, ks, residual, out, part);
+    else if (w0.dtype == VLRF_HIP_DT_Q8_0) launch_dq_split_t<T, VLRF_HIP_DT_Q8_0, EPI>(s, a, w0, w1, M, ks, residual, out, part);
+    else launch_dq_split_t<T, VLRF_HIP_DT_Q4_0, EPI>(s, a, w0, w1, M, ks, residual, out, part);
 }
 
 // out[r][:] = bf16(w ? rmsnorm(x[r]) * w : x[r]), one 256-lane workgroup per row
@@ -1948,8 +1958,8 @@ static bool dq_split_path(const DevWeight& w, int M) { return M >= 17 && M <= 12
 
 size_t qgemm_part_bytes(const DevWeight& w, int M, bool swiglu) {
     int S = 1;
-    if (M > 128) S = big_split_slices(M, w.N, w.K, lds_cus());
-    else if (dq_split_path(w, M)) S = splitk_slices(w, M, swiglu, lds_cus());
+    if (M > 128) S = big_split(M, w.N, w.K, lds_cus()).S;
+    else if (dq_split_path(w, M)) S = mid_split(w, M, swiglu, lds_cus()).S;
     return S > 1 ? (size_t)S * M * w.N * (swiglu ? 2 : 1) * sizeof(float) : 0;
 }
 
@@ -1960,10 +1970,10 @@ int launch_qgemm(hipStream_t s, const DevWeight& w, const uint16_t* a, int M, co
     VH_ARG(a && y, "qgemm: null operand");
     if (M > 128) {
         weight_expand_bf16(s, w);
-        const int S = part ? big_split_slices(M, w.N, w.K, lds_cus()) : 1;
-        if (S > 1 && (w.bf || dqgemm_supported(w))) {
-            if (residual) launch_big_split<1>(s, w.bf != nullptr, a, w, nullptr, M, S, residual, y, part);
-            else launch_big_split<0>(s, w.bf != nullptr, a, w, nullptr, M, S, nullptr, y, part);
+        const KSplit ks = part ? big_split(M, w.N, w.K, lds_cus()) : KSplit{1, w.K};
+        if (ks.S > 1 && (w.bf || dqgemm_supported(w))) {
+            if (residual) launch_big_split<1>(s, w.bf != nullptr, a, w, nullptr, M, ks, residual, y, part);
+            else launch_big_split<0>(s, w.bf != nullptr, a, w, nullptr, M, ks, nullptr, y, part);
         } else if (w.bf) {
             if (residual) launch_bgemm_plan<1>(s, a, w, nullptr, M, residual, y);
             else launch_bgemm_plan<0>(s, a, w, nullptr, M, nullptr, y);
@@ -1976,9 +1986,9 @@ int launch_qgemm(hipStream_t s, const DevWeight& w, const uint16_t* a, int M, co
             else launch_lds_plan<0>(s, p, a, w, nullptr, M, nullptr, y);
         }
     } else if (dq_split_path(w, M) && (part || qgemm_part_bytes(w, M, false) == 0)) {
-        const int S = splitk_slices(w, M, false, lds_cus());
-        if (residual) launch_dq_split<1>(s, a, w, nullptr, M, S, residual, y, part);
-        else launch_dq_split<0>(s, a, w, nullptr, M, S, nullptr, y, part);
+        const KSplit ks = mid_split(w, M, false, lds_cus());
+        if (residual) launch_dq_split<1>(s, a, w, nullptr, M, ks, residual, y, part);
+        else launch_dq_split<0>(s, a, w, nullptr, M, ks, nullptr, y, part);
     } else {
         if (residual) launch_cfg<CfgSmall, 1>(s, w.dtype, a, w, nullptr, M, residual, y);
         else launch_cfg<CfgSmall, 0>(s, w.dtype, a, w, nullptr, M, nullptr, y);
@@ -2003,10 +2013,10 @@ int launch_qgemm_swiglu(hipStream_t s, const DevWeight& wg, const DevWeight& wu,
             (void)hipFree(wg.bf);   // both or neither (no free while capturing)
             wg.bf = nullptr;
         }
-        const int S = part ? big_split_slices(M, wg.N, wg.K, lds_cus()) : 1;
-        if (S > 1 && (both || dqgemm_supported(wg))) {
-            if (h_bf16) launch_big_split<2>(s, both, a, wg, &wu, M, S, nullptr, h, part);
-            else launch_big_split<3>(s, both, a, wg, &wu, M, S, nullptr, h, part);
+        const KSplit ks = part ? big_split(M, wg.N, wg.K, lds_cus()) : KSplit{1, wg.K};
+        if (ks.S > 1 && (both || dqgemm_supported(wg))) {
+            if (h_bf16) launch_big_split<2>(s, both, a, wg, &wu, M, ks, nullptr, h, part);
+            else launch_big_split<3>(s, both, a, wg, &wu, M, ks, nullptr, h, part);
         } else if (both) {
             if (h_bf16) launch_bgemm_plan<2>(s, a, wg, &wu, M, nullptr, h);
             else launch_bgemm_plan<3>(s, a, wg, &wu, M, nullptr, h);
@@ -2019,9 +2029,9 @@ int launch_qgemm_swiglu(hipStream_t s, const DevWeight& wg, const DevWeight& wu,
             else launch_lds_plan<3>(s, p, a, wg, &wu, M, nullptr, h);
         }
     } else if (dq_split_path(wg, M) && (part || qgemm_part_bytes(wg, M, true) == 0)) {
-        const int S = splitk_slices(wg, M, true, lds_cus());
-        if (h_bf16) launch_dq_split<2>(s, a, wg, &wu, M, S, nullptr, h, part);
-        else launch_dq_split<3>(s, a, wg, &wu, M, S, nullptr, h, part);
+        const KSplit ks = mid_split(wg, M, true, lds_cus());
+        if (h_bf16) launch_dq_split<2>(s, a, wg, &wu, M, ks, nullptr, h, part);
+        else launch_dq_split<3>(s, a, wg, &wu, M, ks, nullptr, h, part);
     } else {
         if (h_bf16) launch_cfg<CfgSmall, 2>(s, wg.dtype, a, wg, &wu, M, nullptr, h);
         else launch_cfg<CfgSmall, 3>(s, wg.dtype, a, wg, &wu, M, nullptr, h);
