@@ -1349,6 +1349,22 @@ void launch_dqgemm_plan(hipStream_t s, const uint16_t* a, const DevWeight& w0, c
 // out[r][n] = sum over z of P[z][r][n] (EPI 0), + residual (1, in place
 // allowed), silu(sum of gate) * (sum of up) as bf16 (2) or f32 (3).
 // N % 4 == 0: four columns a thread (VEC), the same sums element by element.
+// Four slices' loads are in flight at a time (one at a time before: 4096 x 14336
+// at M = 20, 14 slices, 27.9 -> 25.5 us; 2048 x 5632, 11 slices, 17.6 -> 16.1),
+// added in slice order.
+__device__ __forceinline__ float4 slice_sum4(const float* __restrict__ p, size_t zs, int S) {
+    float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto add = [&g](float4 t) { g.x += t.x; g.y += t.y; g.z += t.z; g.w += t.w; };
+    auto at = [&](int z) { return *reinterpret_cast<const float4*>(p + z * zs); };
+    int z = 0;
+    for (; z + 4 <= S; z += 4) {
+        const float4 a = at(z), b = at(z + 1), c = at(z + 2), d = at(z + 3);
+        add(a); add(b); add(c); add(d);
+    }
+    for (; z < S; ++z) add(at(z));
+    return g;
+}
+
 template <int EPI>
 __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __restrict__ P, int S, int M, int N,
                                                              int ldp, const float* residual, void* out) {
@@ -1357,17 +1373,9 @@ __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __rest
     const int row = (int)(idx / N), col = (int)(idx % N);
     const size_t zs = (size_t)M * ldp;
     const float* p = P + (size_t)row * ldp + col;
-    float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int z = 0; z < S; ++z) {
-        const float4 t = *reinterpret_cast<const float4*>(p + z * zs);
-        g.x += t.x; g.y += t.y; g.z += t.z; g.w += t.w;
-    }
+    float4 g = slice_sum4(p, zs, S);
     if constexpr (EPI >= 2) {
-        float4 u = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int z = 0; z < S; ++z) {
-            const float4 t = *reinterpret_cast<const float4*>(p + z * zs + N);
-            u.x += t.x; u.y += t.y; u.z += t.z; u.w += t.w;
-        }
+        const float4 u = slice_sum4(p + N, zs, S);
         const float h0 = silu_mul_fast(g.x, u.x), h1 = silu_mul_fast(g.y, u.y);
         const float h2 = silu_mul_fast(g.z, u.z), h3 = silu_mul_fast(g.w, u.w);
         if constexpr (EPI == 2)
