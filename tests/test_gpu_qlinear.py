@@ -162,3 +162,95 @@ def test_qlinear_rejects_bad_shapes(ctx):
         ctx.qlinear(wf, x, ctx.alloc(64 * 4 * 17), 17)     # and a block-quantized weight
     with pytest.raises(V.HipError):
         ctx.qlinear(w, x, x, 1)                             # x aliasing y
+
+
+def _small_bound(x, dec, nw, eps=1e-5):
+    """(y, bound) in 64 bits: f32 sums of K products, exact in pieces, are off by
+    at most (K + 60) eps of the absolute sum; a fused norm adds (K / 2 + 10) eps."""
+    K = x.shape[1]
+    x = x.astype(np.float64)
+    if nw is not None:
+        x = x / np.sqrt((x * x).mean(-1, keepdims=True) + eps) * nw.astype(np.float64)
+    d = dec.astype(np.float64)
+    return x @ d.T, (1.5 * K + 70 if nw is not None else K + 60) * 2.0 ** -24 * (np.abs(x) @ np.abs(d).T)
+
+
+@pytest.mark.parametrize("dtype", [V.DT_Q8_0, V.DT_Q4_0])
+@pytest.mark.parametrize("M,N,K,norm,res", [
+    (16, 64, 128, False, False), (16, 63, 224, True, False), (9, 65, 288, False, True), (2, 130, 1056, True, True),
+    (5, 1, 480, False, False), (3, 700, 1824, True, False), (16, 300, 6176, False, True), (7, 257, 320, True, True),
+    (2, 40, 320, True, False), (4, 64, 14304, False, False)])   # 320 x 2: stays on the vector kernel
+def test_small_m_any_k(ctx, dtype, M, N, K, norm, res):
+    """2..16 rows over K that is no multiple of 256: a last slice of 1..7 blocks,
+    rows of an odd number of blocks, N off the row tile."""
+    print(f"[case] small M any K dtype={dtype} M={M} N={N} K={K} norm={norm} res={res}", flush=True)
+    wf = F.normal(33, f"W{N}x{K}", N * K, 0.02)
+    blocks = F.quantize(wf, dtype)
+    dec = F.dequantize(blocks, dtype, N * K).reshape(N, K)
+    w = V.QuantWeight(ctx, blocks, dtype, N, K)
+    x = F.normal(33, f"x{M}x{K}", M * K).reshape(M, K)
+    nw = 1 + F.normal(33, f"n{K}", K, 0.1) if norm else None
+    r = F.normal(33, f"r{M}x{N}", M * N).reshape(M, N)
+    dy = ctx.to_device(r)
+    ctx.qlinear(w, ctx.to_device(x), dy, M, norm_w=ctx.to_device(nw) if norm else None, residual=dy if res else None)
+    ref, bound = _small_bound(x, dec, nw)
+    if res:
+        ref, bound = ref + r, bound + 2.0 ** -23 * (np.abs(ref) + np.abs(r))
+    assert (np.abs(dy.download((M, N)) - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [V.DT_Q8_0, V.DT_Q4_0])
+@pytest.mark.parametrize("M,N,K", [(16, 70, 352), (3, 200, 1504)])
+def test_small_m_any_k_swiglu_and_specials(ctx, orc, dtype, M, N, K):
+    """SwiGLU over such K; and infinities and NaN in x stay in their rows with the
+    vector kernel's meaning (they have no second and third piece), as does a
+    value whose product with the largest code is still finite."""
+    ws = []
+    for n in "gu":
+        b = F.quantize(F.normal(34, f"{n}{N}x{K}", N * K, 0.02), dtype)
+        ws.append((V.QuantWeight(ctx, b, dtype, N, K), F.dequantize(b, dtype, N * K).reshape(N, K)))
+    x = F.normal(34, f"x{M}x{K}", M * K).reshape(M, K)
+    dh = ctx.alloc(M * N * 4)
+    ctx.qlinear_swiglu(ws[0][0], ws[1][0], ctx.to_device(x), dh, M)
+    ref = orc.silu_mul(orc.linear(x, ws[1][1]), orc.linear(x, ws[0][1]))
+    assert rel_err(dh.download((M, N)), ref) <= 1e-5
+    x[0, K - 1], x[1, 5], x[2] = np.inf, np.nan, 0.0
+    x[2, 7] = 2e36
+    dy = ctx.alloc(M * N * 4)
+    ctx.qlinear(ws[0][0], ctx.to_device(x), dy, M)
+    got, dec = dy.download((M, N)), ws[0][1]
+    last, seven = dec[:, K - 1], dec[:, 7].astype(np.float64) * np.float64(x[2, 7])
+    assert (np.sign(got[0][last != 0]) == np.sign(last[last != 0])).all() and np.isinf(got[0][last != 0]).all()
+    assert np.isnan(got[0][last == 0]).all() and np.isnan(got[1]).all()
+    assert np.allclose(got[2], seven, rtol=1e-6)
+    if M > 3:
+        ref3, bound3 = _small_bound(x[3:], dec, None)
+        assert (np.abs(got[3:] - ref3) <= bound3).all()
+
+
+def test_small_m_any_k_under_graph_capture(orc):
+    """Under capture the call keeps no scratch address: it runs on the vector
+    kernel, and replays to f32 rounding of the eager result, every time."""
+    import ctypes as C
+    from test_gpu_prefill_gemm import _hip
+    hip, ctx = _hip(), V.Context(0)
+    M, N, K = 8, 200, 1056
+    b = F.quantize(F.normal(35, "w", N * K, 0.02), V.DT_Q8_0)
+    w, dec = V.QuantWeight(ctx, b, V.DT_Q8_0, N, K), F.dequantize(b, V.DT_Q8_0, N * K).reshape(N, K)
+    x = F.normal(35, "x", M * K).reshape(M, K)
+    dx, dy, de = ctx.to_device(x), ctx.alloc(M * N * 4), ctx.alloc(M * N * 4)
+    s, g, ge = C.c_void_p(ctx.stream()), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(s, 2) == 0
+    rc = V.lib().vlrf_hip_qlinear(ctx.h, w.h, dx.ptr, dy.ptr, M, None, C.c_float(0.0), None)   # no call before it
+    assert hip.hipStreamEndCapture(s, C.byref(g)) == 0 and rc == 0, V.lib().vlrf_hip_last_error()
+    assert hip.hipGraphInstantiate(C.byref(ge), g, None, None, 0) == 0
+    ref, bound = _small_bound(x, dec, None)
+    for _ in range(3):
+        dy.zero()
+        ctx.qlinear(w, dx, de, M)
+        assert hip.hipGraphLaunch(ge, s) == 0
+        ctx.sync()
+        for d in (dy, de):
+            assert (np.abs(d.download((M, N)) - ref) <= bound).all()
+    hip.hipGraphExecDestroy(ge)
+    hip.hipGraphDestroy(g)

@@ -621,6 +621,22 @@ static int gemm_scratch(Ctx* ctx, size_t a_bytes, size_t p_bytes, float** a, flo
     return p_bytes ? ctx->scratch(a_bytes, a) : rc;
 }
 
+// Scratch of the small-M kernel (2 <= M <= 16); null: the call runs on the vector
+// kernel.  K in whole slices always takes it (an error where the scratch cannot
+// be had); any other K from M K columns of work on, unless the scratch is out
+// of reach (under capture, beyond the tile counters or 2 GiB of partials).  The
+// line, us on the vector kernel / this one at Q8_0: M = 2, 300 x 448 4.3 / 5.2,
+// 14000 x 832 9.2 / 10.4, 14000 x 1344 13.8 / 12.5; M = 3, 300 x 832 6.2 / 5.1; M = 7,
+// 402 x 320 10.2 / 5.4; M = 16, 14000 x 14272 1640 / 84; SwiGLU, M = 2, 14000 x 1344
+// 17.9 / 18.6, 300 x 2112 14.2 / 8.1; M = 16, 5361 x 8000 414 / 35.
+static int small_scratch(Ctx* ctx, const DevWeight& w, int M, bool two, float** out) {
+    const size_t need = qlinear_small_scratch(w.N, w.K, two);
+    if (qlinear_small_whole(w)) return ctx->scratch(need, out);
+    const bool pays = (long)M * w.K >= (two ? 2800 : 1800);
+    *out = pays && qlinear_small_tiles(w.N) <= kSmallMaxTiles && need < 0x7fffffffu ? ctx->try_scratch(need) : nullptr;
+    return VLRF_HIP_OK;
+}
+
 extern "C" {
 
 // M <= 16 runs the f32 GEMV / small-M kernels; larger M (prefill) runs the
@@ -631,13 +647,14 @@ int vlrf_hip_qlinear(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t w, const float* x, fl
     VH_CTX(ctx);
     VH_ARG(w != nullptr, "qlinear: null weight");
     VH_ARG(x != y, "qlinear: x must not alias y");
+    float* scratch_m = nullptr;
     if (M >= 2 && M <= 16 && qlinear_small_supported(w->w)) {
-        float* scratch = nullptr;
-        int rc = ctx->scratch(qlinear_small_scratch(w->w.N, w->w.K, false), &scratch);
+        int rc = small_scratch(ctx, w->w, M, false, &scratch_m);
         if (rc) return rc;
-        return launch_qlinear_small(ctx->stream, w->w, nullptr, x, M, norm_w, eps, residual, scratch,
-                                    ctx->small_tile_ctr, kSmallMaxTiles, y);
     }
+    if (scratch_m)
+        return launch_qlinear_small(ctx->stream, w->w, nullptr, x, M, norm_w, eps, residual, scratch_m,
+                                    ctx->small_tile_ctr, kSmallMaxTiles, y);
     if (M <= 16) return launch_qlinear(ctx->stream, w->w, x, y, M, norm_w, eps, residual);
     VH_ARG(x && y, "qlinear: null activation pointer");
     const size_t a_bytes = ((size_t)M * w->w.K * sizeof(uint16_t) + 255) & ~(size_t)255;
@@ -656,13 +673,14 @@ int vlrf_hip_qlinear_swiglu(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t wg, vlrf_hip_w
     VH_CTX(ctx);
     VH_ARG(wg && wu, "swiglu: null weight");
     VH_ARG(x != h, "swiglu: x must not alias h");
+    float* scratch_m = nullptr;
     if (M >= 2 && M <= 16 && qlinear_small_supported(wg->w)) {
-        float* scratch = nullptr;
-        int rc = ctx->scratch(qlinear_small_scratch(wg->w.N, wg->w.K, true), &scratch);
+        int rc = small_scratch(ctx, wg->w, M, true, &scratch_m);
         if (rc) return rc;
-        return launch_qlinear_small(ctx->stream, wg->w, &wu->w, x, M, norm_w, eps, nullptr, scratch,
-                                    ctx->small_tile_ctr, kSmallMaxTiles, h);
     }
+    if (scratch_m)
+        return launch_qlinear_small(ctx->stream, wg->w, &wu->w, x, M, norm_w, eps, nullptr, scratch_m,
+                                    ctx->small_tile_ctr, kSmallMaxTiles, h);
     if (M <= 16) return launch_qlinear_swiglu(ctx->stream, wg->w, wu->w, x, h, M, norm_w, eps);
     VH_ARG(x && h, "swiglu: null activation pointer");
     const size_t a_bytes = ((size_t)M * wg->w.K * sizeof(uint16_t) + 255) & ~(size_t)255;

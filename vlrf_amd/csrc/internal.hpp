@@ -203,6 +203,7 @@ size_t qgemm_part_bytes(const DevWeight& w, int M, bool swiglu);
 constexpr int kSmallTileCtrStride = 32;   // ints per row-tile counter (its own 128-byte line)
 constexpr int kSmallMaxTiles = 4096;      // row tiles a context's counters cover (N <= 262144 at 64 rows a tile)
 bool qlinear_small_supported(const DevWeight& w);
+bool qlinear_small_whole(const DevWeight& w);   // K in whole slices of 256: no other path takes M = 2..16
 size_t qlinear_small_scratch(int N, int K, bool two);
 int qlinear_small_tiles(int N);
 int launch_qlinear_small(hipStream_t s, const DevWeight& w0, const DevWeight* w1, const float* x,

@@ -1654,7 +1654,22 @@ __device__ __forceinline__ bf16x8 codes_bf16(uint2 c) {
     return r;
 }
 
-template <int WT, int NM, int EPI, int NW>
+// The f32 value as three bf16 pieces of 8 significant bits each, exact: truncated, so
+// that no piece overflows; infinities and NaN stay in the first.
+__device__ __forceinline__ void split3(float v, uint32_t& h, uint32_t& m, uint32_t& l) {
+    const uint32_t u = __float_as_uint(v);
+    const bool fin = (u & 0x7F800000u) != 0x7F800000u;
+    h = fin || !(u & 0x7FFFFFu) ? u & 0xFFFF0000u : 0x7FC00000u;
+    const float r = fin ? v - __uint_as_float(h) : 0.f;
+    m = __float_as_uint(r) & 0xFFFF0000u;
+    l = __float_as_uint(r - __uint_as_float(m)) & 0xFFFF0000u;
+}
+
+// ANY: K any multiple of 32, the last slice with what is left (its missing
+// columns are zeros of x under zero scales), and x in three pieces, so that
+// the products carry all of its 24 bits: those K ran on the f32 vector kernel,
+// whose error against 64 bits (1e-7) two pieces (3e-6) would not keep.
+template <int WT, int NM, int EPI, int NW, bool ANY>
 __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
     const uint8_t* __restrict__ qa, const __half* __restrict__ da, const uint8_t* __restrict__ qb,
     const __half* __restrict__ db, int N, int K, int M, const float* __restrict__ x,
@@ -1666,13 +1681,14 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
     constexpr int CL = 16 * LPR / 64;                    // 16-byte code loads per lane and matrix
     __shared__ __align__(16) uint16_t xh[8 * 16 * 32];
     __shared__ __align__(16) uint16_t xl[8 * 16 * 32];
+    __shared__ __align__(16) uint16_t xm[ANY ? 8 * 16 * 32 : 8];
     __shared__ __align__(16) uint8_t cs[NM][NW][16 * CS];  // per wave: its 16 rows' codes
     __shared__ __align__(16) uint32_t ssc[NM][NW][16 * 4]; // per wave: 16 rows x 8 f16 scales
     constexpr int ROWS = 16 * NW, NI = 512 / (64 * NW);   // rows per workgroup; staging items per thread
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 4, c = lane & 15;
     const int rbase = blockIdx.x * ROWS + 16 * wave;
-    const int ns = K / kSmallSlice;
+    const int ns = (K + kSmallSlice - 1) / kSmallSlice;
     const size_t rowb = WT == VLRF_HIP_DT_Q8_0 ? (size_t)K : (size_t)K / 2;
     // staging: item e = tid + 64 NW i converts row e/32, columns 8(e%32) .. +7 of the slice
     const int sk = 8 * (tid & 31);
@@ -1683,8 +1699,18 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
 #pragma unroll
     for (int m = 0; m < NM; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+    f32x4 sum[NM];   // ANY: over the slices before the current one
+#pragma unroll
+    for (int m = 0; m < NM; ++m) sum[m] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int sl = blockIdx.y; sl < ns; sl += gridDim.y) {
         const int k0 = sl * kSmallSlice;
+        if constexpr (ANY) {
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                sum[m] += acc[m];
+                acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
         // Activations first (L2, needed first), then the codes and scales (HBM):
         // loads complete in order, so the staging below waits for x only.
         float4 a0[NI], a1[NI];
@@ -1692,7 +1718,7 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
         for (int i = 0; i < NI; ++i) {
             const int sm = (tid >> 5) + 2 * NW * i;
             a0[i] = a1[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (sm < M) {
+            if (sm < M && (!ANY || k0 + sk < K)) {
                 const float4* xp = reinterpret_cast<const float4*>(x + (size_t)sm * K + k0 + sk);
                 a0[i] = xp[0];
                 a1[i] = xp[1];
@@ -1709,17 +1735,25 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
 #pragma unroll
             for (int i = 0; i < CL; ++i) {
                 const int r = min(rbase + i * (64 / LPR) + lane / LPR, N - 1);
-                cv[m][i] = *reinterpret_cast<const uint4*>(q + r * rowb + (size_t)k0 * CB / kSmallSlice +
-                                                           16 * (lane % LPR));
+                size_t o = (size_t)k0 * CB / kSmallSlice + 16 * (lane % LPR);
+                if constexpr (ANY) o = o < rowb - 16 ? o : rowb - 16;
+                cv[m][i] = *reinterpret_cast<const uint4*>(q + r * rowb + o);
             }
             const int r = min(rbase + (lane >> 2), N - 1);      // 16 rows x 4 dwords of scales
-            sv[m] = *reinterpret_cast<const uint32_t*>(d + (size_t)r * (K / 32) + k0 / 32 + 2 * (lane & 3));
+            if constexpr (ANY) {                                // rows of any number of blocks: 2-byte loads
+                const uint16_t* dr = reinterpret_cast<const uint16_t*>(d) + (size_t)r * (K / 32);
+                const int b = k0 / 32 + 2 * (lane & 3), nb = K / 32;
+                const uint32_t s0 = dr[min(b, nb - 1)], s1 = dr[min(b + 1, nb - 1)];
+                sv[m] = (b < nb ? s0 : 0u) | (b + 1 < nb ? s1 : 0u) << 16;
+            } else {
+                sv[m] = *reinterpret_cast<const uint32_t*>(d + (size_t)r * (K / 32) + k0 / 32 + 2 * (lane & 3));
+            }
         }
 #pragma unroll
         for (int it = 0; it < NI; ++it) {
             const int sm = (tid >> 5) + 2 * NW * it;
             float4 b0 = a0[it], b1 = a1[it];
-            if (sm < M) {
+            if (sm < M && (!ANY || k0 + sk < K)) {
                 ss[it] += b0.x * b0.x + b0.y * b0.y + b0.z * b0.z + b0.w * b0.w +
                           b1.x * b1.x + b1.y * b1.y + b1.z * b1.z + b1.w * b1.w;
                 if (norm_w) {
@@ -1731,13 +1765,27 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
             }
             const float v[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
             uint32_t h[4], l[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                h[i] = pack_bf16(v[2 * i], v[2 * i + 1]);
-                l[i] = pack_bf16(v[2 * i] - __uint_as_float(h[i] << 16),
-                                 v[2 * i + 1] - __uint_as_float(h[i] & 0xFFFF0000u));
-            }
             const int o = (sk >> 5) * 512 + sm * 32 + (sk & 31);
+            if constexpr (ANY) {
+                uint32_t md[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    uint32_t h0, m0, l0, h1, m1, l1;
+                    split3(v[2 * i], h0, m0, l0);
+                    split3(v[2 * i + 1], h1, m1, l1);
+                    h[i] = h0 >> 16 | h1;
+                    md[i] = m0 >> 16 | m1;
+                    l[i] = l0 >> 16 | l1;
+                }
+                *reinterpret_cast<uint4*>(xm + o) = make_uint4(md[0], md[1], md[2], md[3]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    h[i] = pack_bf16(v[2 * i], v[2 * i + 1]);
+                    l[i] = pack_bf16(v[2 * i] - __uint_as_float(h[i] << 16),
+                                     v[2 * i + 1] - __uint_as_float(h[i] & 0xFFFF0000u));
+                }
+            }
             *reinterpret_cast<uint4*>(xh + o) = make_uint4(h[0], h[1], h[2], h[3]);
             *reinterpret_cast<uint4*>(xl + o) = make_uint4(l[0], l[1], l[2], l[3]);
         }
@@ -1763,8 +1811,16 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
                 else
                     code = make_uint2(*reinterpret_cast<const uint32_t*>(&cs[m][wave][c * CS + 16 * j + 4 * g]), 0u);
                 const bf16x8 a = codes_bf16<WT>(code);
-                f32x4 t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bh, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bl, t, 0, 0, 0);
+                f32x4 t;
+                if constexpr (ANY) {   // the small pieces first
+                    const bf16x8 bm = *reinterpret_cast<const bf16x8*>(xm + xo);
+                    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bl, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bm, t, 0, 0, 0);
+                    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bh, t, 0, 0, 0);
+                } else {
+                    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bh, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bl, t, 0, 0, 0);
+                }
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const uint32_t wd = ssc[m][wave][(4 * g + v) * 4 + (j >> 1)];
@@ -1776,6 +1832,10 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
         __syncthreads();                      // before the next slice overwrites the staging
     }
 
+    if constexpr (ANY) {
+#pragma unroll
+        for (int m = 0; m < NM; ++m) acc[m] += sum[m];
+    }
     // This slice's partials, device-coherent (the tile's last workgroup may
     // run on another XCD): columns m < M only.
     const int S = gridDim.y;
@@ -1874,7 +1934,7 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
 // once) up to about 1024 workgroups (4 per CU); beyond that columns take
 // several slices, which bounds the partial-sum scratch.
 int small_grid_y(int N, int K, int rows) {
-    const int groups = (N + rows - 1) / rows, ns = K / kSmallSlice;
+    const int groups = (N + rows - 1) / rows, ns = (K + kSmallSlice - 1) / kSmallSlice;
     const int want = (1024 + groups - 1) / groups;
     return want < ns ? want : ns;
 }
@@ -2049,8 +2109,12 @@ int launch_qgemm_swiglu(hipStream_t s, const DevWeight& wg, const DevWeight& wu,
 }
 
 bool qlinear_small_supported(const DevWeight& w) {
-    return (w.dtype == VLRF_HIP_DT_Q8_0 || w.dtype == VLRF_HIP_DT_Q4_0) && w.q && w.d && w.K % kSmallSlice == 0;
+    return (w.dtype == VLRF_HIP_DT_Q8_0 || w.dtype == VLRF_HIP_DT_Q4_0) && w.q && w.d && w.K % 32 == 0;
 }
+
+// K in whole slices: the form that needs its scratch and counters; any other K
+// can also run without them (launch_qlinear).
+bool qlinear_small_whole(const DevWeight& w) { return w.K % kSmallSlice == 0; }
 
 int qlinear_small_tiles(int N) { const int rows = 16 * small_waves(); return (N + rows - 1) / rows; }
 
@@ -2078,24 +2142,29 @@ int launch_qlinear_small(hipStream_t s, const DevWeight& w0, const DevWeight* w1
     const dim3 grid(qlinear_small_tiles(N), S);
     const uint8_t* qb = w1 ? w1->q : nullptr;
     const __half* db = w1 ? w1->d : nullptr;
-#define VH_SMALL(WT, NMV, EPIV)                                                                                 \
-    do {                                                                                                        \
-        if (NW == 8)                                                                                            \
-            hipLaunchKernelGGL((qlinear_small_kernel<WT, NMV, EPIV, 8>), grid, dim3(512), 0, s, w0.q, w0.d, qb, \
-                               db, N, K, M, x, norm_w, eps, residual, y, P, SS, tile_ctr);                      \
-        else                                                                                                    \
-            hipLaunchKernelGGL((qlinear_small_kernel<WT, NMV, EPIV, 4>), grid, dim3(256), 0, s, w0.q, w0.d, qb, \
-                               db, N, K, M, x, norm_w, eps, residual, y, P, SS, tile_ctr);                      \
+#define VH_SMALL(WT, NMV, EPIV, NWV, ANYV)                                                                      \
+    hipLaunchKernelGGL((qlinear_small_kernel<WT, NMV, EPIV, NWV, ANYV>), grid, dim3(64 * NWV), 0, s, w0.q, w0.d, \
+                       qb, db, N, K, M, x, norm_w, eps, residual, y, P, SS, tile_ctr)
+#define VH_SMALL_K(WT, NMV, EPIV)                                      \
+    do {                                                               \
+        if (qlinear_small_whole(w0)) {                                 \
+            if (NW == 8) VH_SMALL(WT, NMV, EPIV, 8, false);            \
+            else VH_SMALL(WT, NMV, EPIV, 4, false);                    \
+        } else {                                                       \
+            if (NW == 8) VH_SMALL(WT, NMV, EPIV, 8, true);             \
+            else VH_SMALL(WT, NMV, EPIV, 4, true);                     \
+        }                                                              \
     } while (0)
-#define VH_SMALL_T(WT)                                         \
-    do {                                                       \
-        if (w1) VH_SMALL(WT, 2, 3);                            \
-        else if (residual) VH_SMALL(WT, 1, 1);                 \
-        else VH_SMALL(WT, 1, 0);                               \
+#define VH_SMALL_T(WT)                                           \
+    do {                                                         \
+        if (w1) VH_SMALL_K(WT, 2, 3);                            \
+        else if (residual) VH_SMALL_K(WT, 1, 1);                 \
+        else VH_SMALL_K(WT, 1, 0);                               \
     } while (0)
     if (w0.dtype == VLRF_HIP_DT_Q8_0) VH_SMALL_T(VLRF_HIP_DT_Q8_0);
     else VH_SMALL_T(VLRF_HIP_DT_Q4_0);
 #undef VH_SMALL_T
+#undef VH_SMALL_K
 #undef VH_SMALL
     VH_LAUNCHED();
     return VLRF_HIP_OK;
