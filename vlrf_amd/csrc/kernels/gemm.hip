@@ -1430,21 +1430,23 @@ void launch_splitk_reduce(hipStream_t s, const float* part, int S, int M, int N,
 using SplitTile64 = BTile<64, 256, 2, 4>;     // M <= 64: 8 waves of 32 x 64
 using SplitTile128 = BTile<128, 128, 4, 2>;   // 65 <= M <= 128: 8 waves of 32 x 64
 
-// A split of K's steps of 64: S slices of kl columns, the last one with what is left.
+// A split of K's steps of 64: S slices of kl columns, the last one with what is
+// left; over the half-size tiles (few) or the plan's own.
 struct KSplit {
     int S, kl;
+    bool few = false;
 };
 
 // As many slices as fit one round of the CUs beside each other (tiles output
-// tiles), of at least 8 steps: a number down to 3/4 of that which divides the
+// tiles), of at least `least` steps: a number down to 3/4 of that which divides the
 // steps, if there is one (8B QKV at M = 100, 48 tiles of 64 steps: 4 slices 23.9
 // us, 5 uneven ones 24.4), else that many, as even as whole steps allow.  (us at
 // Q8_0, slices that had to divide K / 128 or none -> these: 4123 x 10944, M = 105,
 // 221 -> 33.5; 2048 x 5504, M = 128, 60 -> 22; 4757 x 9856, M = 395, 122 -> 79;
 // 773 x 10432, M = 20, 191 -> 21.6.)
-KSplit split_k(long tiles, int K, int cus) {
+KSplit split_k(long tiles, int K, int cus, int least = 8) {
     const int steps = K / 64;
-    long S = cus / tiles < steps / 8 ? cus / tiles : steps / 8;
+    long S = cus / tiles < steps / least ? cus / tiles : steps / least;
     if (S < 1) S = 1;
     for (long d = S; 4 * d >= 3 * S; --d)
         if (steps % d == 0) {
@@ -1455,12 +1457,36 @@ KSplit split_k(long tiles, int K, int cus) {
     return {(steps + per - 1) / per, per * 64};
 }
 
-KSplit mid_split(const DevWeight& w, int M, bool swiglu, int cus) {
-    const int bn = (M <= 64 ? SplitTile64::BN : SplitTile128::BN) / (swiglu ? 2 : 1);
-    return split_k((w.N + bn - 1) / bn, w.K, cus);
+// Where the plan's tiles and slices fill at most half of the CUs (small N or
+// short K), tiles of half the columns and, above 128 rows, half the rows, four
+// waves and three stages of A each, in at most 24 slices of at least 4 steps:
+// more and shorter workgroups.  Two slices of up to 16 steps do not pay for their
+// reduction, nor small tiles for their operands beyond 2.5 rounds.  us, the
+// plan's tiles / these: 1236 x 1344, M = 38, 15.5 / 11.0; 345 x 1216, M = 324, 17.0 /
+// 12.1; 2270 x 1216, M = 434, 22.9 / 15.7; 1.1B QKV and O at M = 233 21.7 / 17.9, 20.0 /
+// 16.6; SwiGLU 383 x 1152, M = 202, 21.4 / 12.3.  At more than half a round: 8B QKV,
+// M = 100, 25.0 / 25.3; 8B down, M = 400, 90 / 111.
+using FewTile64 = BTile<64, 128, 2, 2>;
+using FewTile128 = BTile<128, 64, 4, 1>;
+
+KSplit few_split(const DevWeight& w, int M, bool swiglu, const KSplit& own, long tiles, int cus) {
+    if (2 * tiles * own.S > cus || !dqgemm_supported(w)) return own;
+    const int bm = M <= 64 ? FewTile64::BM : FewTile128::BM, bn = (M <= 64 ? FewTile64::BN : FewTile128::BN) / (swiglu ? 2 : 1);
+    const long few = (long)((M + bm - 1) / bm) * ((w.N + bn - 1) / bn);
+    if (2 * few > 5L * cus) return own;
+    KSplit ks = split_k(few, w.K, cus < 24 * few ? cus : (int)(24 * few), 4);
+    if (ks.S == 2 && w.K <= 16 * 64) ks = {1, w.K};
+    ks.few = true;
+    return ks;
 }
 
-template <class T, int WT, int EPI>
+KSplit mid_split(const DevWeight& w, int M, bool swiglu, int cus) {
+    const int bn = (M <= 64 ? SplitTile64::BN : SplitTile128::BN) / (swiglu ? 2 : 1);
+    const long nt = (w.N + bn - 1) / bn;
+    return few_split(w, M, swiglu, split_k(nt, w.K, cus), nt, cus);
+}
+
+template <class T, int WT, int EPI, int NSA = 2>
 void launch_dq_split_t(hipStream_t s, const uint16_t* a, const DevWeight& w0, const DevWeight* w1, int M, KSplit ks,
                        const float* residual, void* out, float* part) {
     constexpr bool SW = EPI >= 2;
@@ -1470,19 +1496,31 @@ void launch_dq_split_t(hipStream_t s, const uint16_t* a, const DevWeight& w0, co
     const uint8_t* qb = SW ? w1->q : w0.q;
     const __half* db = SW ? w1->d : w0.d;
     if (ks.S == 1) {
-        hipLaunchKernelGGL((mfma_dqgemm_kernel<T, WT, EPI, 2>), grid, dim3(T::NT), 0, s, a, w0.q, w0.d, qb, db, M, N,
+        hipLaunchKernelGGL((mfma_dqgemm_kernel<T, WT, EPI, NSA>), grid, dim3(T::NT), 0, s, a, w0.q, w0.d, qb, db, M, N,
                            K, K, N, residual, out);
         return;
     }
     const int ldp = SW ? 2 * N : N;
-    hipLaunchKernelGGL((mfma_dqgemm_kernel<T, WT, SW ? 7 : 6, 2>), grid, dim3(T::NT), 0, s, a, w0.q, w0.d, qb, db, M,
+    hipLaunchKernelGGL((mfma_dqgemm_kernel<T, WT, SW ? 7 : 6, NSA>), grid, dim3(T::NT), 0, s, a, w0.q, w0.d, qb, db, M,
                        N, K, ks.kl, ldp, nullptr, part);
     launch_splitk_reduce<EPI>(s, part, ks.S, M, N, ldp, residual, out);
+}
+
+template <int WT, int EPI>
+void launch_few(hipStream_t s, const uint16_t* a, const DevWeight& w0, const DevWeight* w1, int M, KSplit ks,
+                const float* residual, void* out, float* part) {
+    if (M <= 64) launch_dq_split_t<FewTile64, WT, EPI, 3>(s, a, w0, w1, M, ks, residual, out, part);
+    else launch_dq_split_t<FewTile128, WT, EPI, 3>(s, a, w0, w1, M, ks, residual, out, part);
 }
 
 template <int EPI>
 void launch_dq_split(hipStream_t s, const uint16_t* a, const DevWeight& w0, const DevWeight* w1, int M, KSplit ks,
                      const float* residual, void* out, float* part) {
+    if (ks.few) {
+        if (w0.dtype == VLRF_HIP_DT_Q8_0) launch_few<VLRF_HIP_DT_Q8_0, EPI>(s, a, w0, w1, M, ks, residual, out, part);
+        else launch_few<VLRF_HIP_DT_Q4_0, EPI>(s, a, w0, w1, M, ks, residual, out, part);
+        return;
+    }
     if (w0.dtype == VLRF_HIP_DT_Q8_0) {
         if (M <= 64) launch_dq_split_t<SplitTile64, VLRF_HIP_DT_Q8_0, EPI>(s, a, w0, w1, M, ks, residual, out, part);
         else launch_dq_split_t<SplitTile128, VLRF_HIP_DT_Q8_0, EPI>(s, a, w0, w1, M, ks, residual, out, part);
@@ -1503,11 +1541,11 @@ void launch_dq_split(hipStream_t s, const uint16_t* a, const DevWeight& w0, cons
 // (8B layer, same box: against aiming at 3/4 of a round from below half a
 // round, T = 1024 0.677 -> 0.600 ms, its O and down now split in two; T =
 // 256 .. 768 within noise.  Aiming at a full round: T = 256 0.291 ms.)
-KSplit big_split(int M, int N, int K, int cus) {
-    const long g0 = (long)((M + 255) / 256) * ((N + 127) / 128);
+KSplit big_split(const DevWeight& w, int M, bool swiglu, int cus) {
+    const long g0 = (long)((M + 255) / 256) * ((w.N + 127) / 128);
     const char* e = getenv("VLRF_HIP_PREFILL_SPLIT");   // "0": the unsplit plans at every M > 128
-    if ((e && e[0] == '0') || g0 >= cus) return {1, K};
-    return split_k(g0, K, cus);
+    if ((e && e[0] == '0') || g0 >= cus) return {1, w.K};
+    return few_split(w, M, swiglu, split_k(g0, w.K, cus), g0, cus);
 }
 
 template <class T, int EPI>
@@ -2026,7 +2064,7 @@ static bool dq_split_path(const DevWeight& w, int M) { return M >= 17 && M <= 12
 
 size_t qgemm_part_bytes(const DevWeight& w, int M, bool swiglu) {
     int S = 1;
-    if (M > 128) S = big_split(M, w.N, w.K, lds_cus()).S;
+    if (M > 128) S = big_split(w, M, swiglu, lds_cus()).S;
     else if (dq_split_path(w, M)) S = mid_split(w, M, swiglu, lds_cus()).S;
     return S > 1 ? (size_t)S * M * w.N * (swiglu ? 2 : 1) * sizeof(float) : 0;
 }
@@ -2038,8 +2076,11 @@ int launch_qgemm(hipStream_t s, const DevWeight& w, const uint16_t* a, int M, co
     VH_ARG(a && y, "qgemm: null operand");
     if (M > 128) {
         weight_expand_bf16(s, w);
-        const KSplit ks = part ? big_split(M, w.N, w.K, lds_cus()) : KSplit{1, w.K};
-        if (ks.S > 1 && (w.bf || dqgemm_supported(w))) {
+        const KSplit ks = part || !qgemm_part_bytes(w, M, false) ? big_split(w, M, false, lds_cus()) : KSplit{1, w.K};
+        if (ks.few) {
+            if (residual) launch_dq_split<1>(s, a, w, nullptr, M, ks, residual, y, part);
+            else launch_dq_split<0>(s, a, w, nullptr, M, ks, nullptr, y, part);
+        } else if (ks.S > 1 && (w.bf || dqgemm_supported(w))) {
             if (residual) launch_big_split<1>(s, w.bf != nullptr, a, w, nullptr, M, ks, residual, y, part);
             else launch_big_split<0>(s, w.bf != nullptr, a, w, nullptr, M, ks, nullptr, y, part);
         } else if (w.bf) {
@@ -2081,8 +2122,11 @@ int launch_qgemm_swiglu(hipStream_t s, const DevWeight& wg, const DevWeight& wu,
             (void)hipFree(wg.bf);   // both or neither (no free while capturing)
             wg.bf = nullptr;
         }
-        const KSplit ks = part ? big_split(M, wg.N, wg.K, lds_cus()) : KSplit{1, wg.K};
-        if (ks.S > 1 && (both || dqgemm_supported(wg))) {
+        const KSplit ks = part || !qgemm_part_bytes(wg, M, true) ? big_split(wg, M, true, lds_cus()) : KSplit{1, wg.K};
+        if (ks.few) {
+            if (h_bf16) launch_dq_split<2>(s, a, wg, &wu, M, ks, nullptr, h, part);
+            else launch_dq_split<3>(s, a, wg, &wu, M, ks, nullptr, h, part);
+        } else if (ks.S > 1 && (both || dqgemm_supported(wg))) {
             if (h_bf16) launch_big_split<2>(s, both, a, wg, &wu, M, ks, nullptr, h, part);
             else launch_big_split<3>(s, both, a, wg, &wu, M, ks, nullptr, h, part);
         } else if (both) {
