@@ -159,3 +159,38 @@ def test_gelu_and_add(ctx, orc, n):
     a, b = ctx.to_device(x), ctx.to_device(y)
     ctx.add(a, b, n)
     assert np.array_equal(a.download(x.shape), x + y)       # one rounding per element, as the CPU
+
+
+@pytest.mark.parametrize("n,off", [(3, 0), (4, 0), (5, 1), (1023, 0), (4099, 2), (70003, 0)])
+def test_gelu_and_add_groups_of_four(ctx, orc, n, off):
+    """Counts off the groups of four and addresses off 16 bytes: the same values as
+    element by element, nothing beyond the end written."""
+    x, y = F.normal(67, f"x{n}", n) * 3, F.normal(67, f"y{n}", n)
+    pad = np.full(off, 9.0, np.float32)
+    a, b = (ctx.to_device(np.concatenate([pad, t, pad, [9.0]]).astype(np.float32)) for t in (x, y))
+    V.check(V.lib().vlrf_hip_gelu(ctx.h, a.ptr + 4 * off, n))
+    g = a.download((n + 2 * off + 1,))
+    assert rel_err(g[off:off + n], orc.gelu(x)) <= 1e-6
+    V.check(V.lib().vlrf_hip_add(ctx.h, a.ptr + 4 * off, b.ptr + 4 * off, n))
+    s = a.download((n + 2 * off + 1,))
+    assert np.array_equal(s[off:off + n], g[off:off + n] + y)
+    assert (np.delete(s, np.s_[off:off + n]) == 9.0).all() and (np.delete(g, np.s_[off:off + n]) == 9.0).all()
+
+
+@pytest.mark.parametrize("rows,D,off", [(5, 4, 0), (3, 1020, 0), (2, 1028, 0), (2, 4096, 0), (2, 4100, 0), (3, 768, 1)])
+def test_layer_norm_in_registers(ctx, rows, D, off):
+    """Row lengths at the edges of the register form, and addresses that forbid it,
+    against 64 bits: every step is an f32 sum of D terms."""
+    x = F.normal(68, f"x{D}", rows * D).reshape(rows, D) * 2 + 1
+    w, b = 1 + F.normal(68, f"w{D}", D, 0.1), F.normal(68, f"b{D}", D, 0.1)
+    pad = np.zeros(off, np.float32)
+    dx, dw, db = (ctx.to_device(np.concatenate([pad, t.ravel()]).astype(np.float32)) for t in (x, w, b))
+    do = ctx.alloc(4 * (rows * D + off))
+    V.check(V.lib().vlrf_hip_layer_norm(ctx.h, *[t.ptr + 4 * off for t in (dx, dw, db, do)], rows, D, 1e-5))
+    got = do.download((rows * D + off,))[off:].reshape(rows, D)
+    x64 = x.astype(np.float64)
+    c = x64 - x64.mean(1, keepdims=True)
+    inv = 1 / np.sqrt((c * c).mean(1, keepdims=True) + 1e-5)
+    ref = c * inv * w + b
+    bound = (D + 20) * 2.0 ** -24 * (np.abs(x64).max() * inv * np.abs(w) + np.abs(ref) + np.abs(b))
+    assert (np.abs(got - ref) <= bound).all()

@@ -232,6 +232,47 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const float* __restrict
     for (int j = threadIdx.x; j < D; j += 256) o[j] = (r[j] - mean) * inv * w[j] + b[j];
 }
 
+// Rows of up to 4096 columns held in registers, four float4 a thread: read once, and
+// no load behind a reduction (a call among others, 1000 x 1600: 5.3 -> 4.4 us; 300 x 768
+// 3.7 -> 3.5, near what a launch costs).
+__global__ __launch_bounds__(256) void layer_norm_regs_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                              const float* __restrict__ b, float* out, int D,
+                                                              float eps) {
+    __shared__ float red[4];
+    const float4* r = reinterpret_cast<const float4*>(x + (size_t)blockIdx.x * D);
+    const int n4 = D / 4;
+    float4 v[4], wv[4], bv[4];
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int j = min((int)threadIdx.x + 256 * i, n4 - 1);
+        v[i] = r[j];
+        wv[i] = reinterpret_cast<const float4*>(w)[j];
+        bv[i] = reinterpret_cast<const float4*>(b)[j];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if ((int)threadIdx.x + 256 * i < n4) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+    const float mean = block_sum(s, red) / (float)D;
+    float q = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        v[i] = make_float4(v[i].x - mean, v[i].y - mean, v[i].z - mean, v[i].w - mean);
+        if ((int)threadIdx.x + 256 * i < n4)
+            q += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+    }
+    const float var = block_sum(q, red) / (float)D + eps;
+    const float inv = 1.f / sqrtf(var);
+    float4* o = reinterpret_cast<float4*>(out + (size_t)blockIdx.x * D);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int j = threadIdx.x + 256 * i;
+        if (j < n4)
+            o[j] = make_float4(v[i].x * inv * wv[i].x + bv[i].x, v[i].y * inv * wv[i].y + bv[i].y,
+                               v[i].z * inv * wv[i].z + bv[i].z, v[i].w * inv * wv[i].w + bv[i].w);
+    }
+}
+
 __global__ __launch_bounds__(256) void softmax_kernel(float* x, int D) {
     __shared__ float red[4];
     float* r = x + (size_t)blockIdx.x * D;
@@ -248,18 +289,36 @@ __global__ __launch_bounds__(256) void softmax_kernel(float* x, int D) {
     for (int j = threadIdx.x; j < D; j += 256) r[j] *= inv;
 }
 
-__global__ __launch_bounds__(256) void gelu_kernel(float* x, int64_t n) {
+__device__ __forceinline__ float gelu_tanh(float v) {
     constexpr float c1 = 0.7978845608028654f, c2 = 0.044715f;   // sqrt(2/pi), ops.hpp:393-394
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-        const float v = x[i];
-        const float inner = c1 * (v + c2 * v * v * v);
-        x[i] = 0.5f * v * (1.f + tanhf(inner));
-    }
+    const float inner = c1 * (v + c2 * v * v * v);
+    return 0.5f * v * (1.f + tanhf(inner));
 }
 
+// VEC: 16-byte accesses over whole groups of four (aligned bases), the rest singly
+// (1000 x 6400: 7.9 -> 6.8 us; add of 1000 x 1600 3.9 -> 3.4).
+template <bool VEC>
+__global__ __launch_bounds__(256) void gelu_kernel(float* x, int64_t n) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256, n4 = VEC ? n / 4 : 0;
+    for (int64_t i = t; i < n4; i += step) {
+        const float4 v = reinterpret_cast<const float4*>(x)[i];
+        reinterpret_cast<float4*>(x)[i] = make_float4(gelu_tanh(v.x), gelu_tanh(v.y), gelu_tanh(v.z), gelu_tanh(v.w));
+    }
+    for (int64_t i = 4 * n4 + t; i < n; i += step) x[i] = gelu_tanh(x[i]);
+}
+
+template <bool VEC>
 __global__ __launch_bounds__(256) void add_kernel(float* dst, const float* __restrict__ src, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
-        dst[i] += src[i];
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256, n4 = VEC ? n / 4 : 0;
+    for (int64_t i = t; i < n4; i += step) {
+        const float4 d = reinterpret_cast<const float4*>(dst)[i], s = reinterpret_cast<const float4*>(src)[i];
+        reinterpret_cast<float4*>(dst)[i] = make_float4(d.x + s.x, d.y + s.y, d.z + s.z, d.w + s.w);
+    }
+    for (int64_t i = 4 * n4 + t; i < n; i += step) dst[i] += src[i];
+}
+
+bool aligned16(const void* a, const void* b = nullptr, const void* c = nullptr, const void* d = nullptr) {
+    return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d) & 15) == 0;
 }
 
 int grid_1d(int64_t n) {
@@ -362,7 +421,10 @@ int launch_gemm_f32(hipStream_t s, const float* A, const float* B, float* C, int
 int launch_layer_norm(hipStream_t s, const float* x, const float* w, const float* b, float* out, int rows, int D,
                       float eps) {
     VH_ARG(x && w && b && out && rows >= 1 && D >= 1, "layer_norm: bad arguments");
-    hipLaunchKernelGGL(layer_norm_kernel, dim3(rows), dim3(256), 0, s, x, w, b, out, D, eps);
+    if (D % 4 == 0 && D <= 4096 && aligned16(x, w, b, out))
+        hipLaunchKernelGGL(layer_norm_regs_kernel, dim3(rows), dim3(256), 0, s, x, w, b, out, D, eps);
+    else
+        hipLaunchKernelGGL(layer_norm_kernel, dim3(rows), dim3(256), 0, s, x, w, b, out, D, eps);
     VH_LAUNCHED();
     return VLRF_HIP_OK;
 }
@@ -377,7 +439,8 @@ int launch_softmax(hipStream_t s, float* x, int rows, int D) {
 int launch_gelu(hipStream_t s, float* x, int64_t n) {
     VH_ARG(x && n >= 0, "gelu: bad arguments");
     if (n == 0) return VLRF_HIP_OK;
-    hipLaunchKernelGGL(gelu_kernel, dim3(grid_1d(n)), dim3(256), 0, s, x, n);
+    if (aligned16(x)) hipLaunchKernelGGL((gelu_kernel<true>), dim3(grid_1d((n + 3) / 4)), dim3(256), 0, s, x, n);
+    else hipLaunchKernelGGL((gelu_kernel<false>), dim3(grid_1d(n)), dim3(256), 0, s, x, n);
     VH_LAUNCHED();
     return VLRF_HIP_OK;
 }
@@ -385,7 +448,8 @@ int launch_gelu(hipStream_t s, float* x, int64_t n) {
 int launch_add(hipStream_t s, float* dst, const float* src, int64_t n) {
     VH_ARG(dst && src && n >= 0, "add: bad arguments");
     if (n == 0) return VLRF_HIP_OK;
-    hipLaunchKernelGGL(add_kernel, dim3(grid_1d(n)), dim3(256), 0, s, dst, src, n);
+    if (aligned16(dst, src)) hipLaunchKernelGGL((add_kernel<true>), dim3(grid_1d((n + 3) / 4)), dim3(256), 0, s, dst, src, n);
+    else hipLaunchKernelGGL((add_kernel<false>), dim3(grid_1d(n)), dim3(256), 0, s, dst, src, n);
     VH_LAUNCHED();
     return VLRF_HIP_OK;
 }
