@@ -59,6 +59,8 @@ struct vlrf_hip_model {
     DevWeight lm_head;
     bool embed_set = false, ln_final_set = false, lm_head_set = false;
     std::vector<Layer> layers;
+    int8_t* kv_all = nullptr;   // the layers' caches (Layer::kv points into it)
+    size_t kv_bytes = 0;
     const float* cos_t = nullptr;
     const float* sin_t = nullptr;
     float *x = nullptr, *qkv = nullptr, *att = nullptr, *h = nullptr, *logits = nullptr, *part = nullptr;
@@ -411,16 +413,26 @@ int vlrf_hip_model_create(vlrf_hip_ctx_t ctx, const vlrf_hip_model_config* cfg, 
     dalloc((void**)&m->state, 4 * sizeof(int));
     dalloc((void**)&m->gen_ids, (size_t)m->S * sizeof(int));
     dalloc((void**)&m->prompt, (size_t)m->S * sizeof(int));
-    const size_t kvdata = (size_t)m->G * m->S * dh * kv_elem_bytes(c.kv_dtype);
+    // Every layer's K, V and row scales in one allocation (each on its own 256
+    // bytes), so that a reset clears them in one go.
+    auto up256 = [](size_t n) { return (n + 255) & ~(size_t)255; };
+    const size_t kvdata = up256((size_t)m->G * m->S * dh * kv_elem_bytes(c.kv_dtype));
+    const size_t kvscales = c.kv_dtype == VLRF_HIP_KV_Q8_0 ? up256((size_t)m->S * 4) : 0;
+    m->kv_bytes = 2 * (kvdata + kvscales) * m->L;
+    dalloc((void**)&m->kv_all, m->kv_bytes);
+    int8_t* kv_at = m->kv_all;
     for (auto& Ly : m->layers) {
         dalloc((void**)&Ly.ln1, (size_t)m->D * 4);
         dalloc((void**)&Ly.ln2, (size_t)m->D * 4);
         Ly.kv.dtype = c.kv_dtype;
-        dalloc((void**)&Ly.kv.k, kvdata);
-        dalloc((void**)&Ly.kv.v, kvdata);
-        if (c.kv_dtype == VLRF_HIP_KV_Q8_0) {
-            dalloc((void**)&Ly.kv.ks, (size_t)m->S * 4);
-            dalloc((void**)&Ly.kv.vs, (size_t)m->S * 4);
+        if (!rc) {
+            Ly.kv.k = kv_at;
+            Ly.kv.v = kv_at + kvdata;
+            if (kvscales) {
+                Ly.kv.ks = reinterpret_cast<float*>(kv_at + 2 * kvdata);
+                Ly.kv.vs = reinterpret_cast<float*>(kv_at + 2 * kvdata + kvscales);
+            }
+            kv_at += 2 * (kvdata + kvscales);
         }
         if (!rc) rc = weight_alloc(Ly.wqkv, c.weight_dtype, m->D + 2 * m->dkv, m->D);
         if (!rc) rc = weight_alloc(Ly.wo, c.weight_dtype, m->D, m->D);
@@ -456,8 +468,7 @@ void vlrf_hip_model_destroy(vlrf_hip_model_t m) {
     (void)hipStreamSynchronize(m->ctx->stream);
     drop_graphs(m);
     for (auto& Ly : m->layers) {
-        for (void* p : {(void*)Ly.ln1, (void*)Ly.ln2, (void*)Ly.kv.k, (void*)Ly.kv.v, (void*)Ly.kv.ks,
-                        (void*)Ly.kv.vs})
+        for (void* p : {(void*)Ly.ln1, (void*)Ly.ln2})
             if (p) (void)hipFree(p);
         weight_release(Ly.wqkv);
         weight_release(Ly.wo);
@@ -468,7 +479,7 @@ void vlrf_hip_model_destroy(vlrf_hip_model_t m) {
     weight_release(m->lm_head);
     for (void* p : {(void*)m->embed, (void*)m->ln_final, (void*)m->x, (void*)m->qkv, (void*)m->att,
                     (void*)m->h, (void*)m->logits, (void*)m->argpairs, (void*)m->part, (void*)m->chunks, (void*)m->state,
-                    (void*)m->gen_ids, (void*)m->prompt})
+                    (void*)m->gen_ids, (void*)m->prompt, (void*)m->kv_all})
         if (p) (void)hipFree(p);
     for (void* p : {(void*)m->pf_x, (void*)m->pf_qkv, (void*)m->pf_a, (void*)m->pf_att, (void*)m->pf_h,
                     (void*)m->pf_ids, (void*)m->pf_part, (void*)m->qkv_tags,
@@ -554,13 +565,9 @@ int vlrf_hip_model_reset(vlrf_hip_model_t m) {
     VH_ARG(m != nullptr, "model_reset: null handle");
     VH_CHECK(hipSetDevice(m->ctx->device));
     hipStream_t s = m->ctx->stream;
-    const size_t kvdata = (size_t)m->G * m->S * m->dh * kv_elem_bytes(m->cfg.kv_dtype);
-    for (auto& Ly : m->layers) {
-        VH_CHECK(hipMemsetAsync(Ly.kv.k, 0, kvdata, s));
-        VH_CHECK(hipMemsetAsync(Ly.kv.v, 0, kvdata, s));
-        if (Ly.kv.ks) VH_CHECK(hipMemsetAsync(Ly.kv.ks, 0, (size_t)m->S * 4, s));
-        if (Ly.kv.vs) VH_CHECK(hipMemsetAsync(Ly.kv.vs, 0, (size_t)m->S * 4, s));
-    }
+    // One clear for all layers: a launch for each layer's K, V and scales took
+    // 0.2 ms of a 22-layer model's request.
+    VH_CHECK(hipMemsetAsync(m->kv_all, 0, m->kv_bytes, s));
     VH_CHECK(hipMemsetAsync(m->state, 0, 3 * sizeof(int), s));   // the epoch (state[3]) runs on
     VH_CHECK(hipStreamSynchronize(s));
     m->pos = 0;
