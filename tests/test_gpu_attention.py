@@ -86,6 +86,21 @@ def test_sdp_attention_tiles(ctx, T, ctx_len, d, causal, scale, off):
     assert (got[Q.size:] == 7.0).all()
 
 
+def test_sdp_attention_long_grid(ctx):
+    """More blocks of queries than a grid takes along y: 2^20 queries a z step,
+    past 65535 blocks, a ragged last one.  One key: the result is its value."""
+    T, d = 65535 * 32 + 45, 4
+    print(f"[case] sdp long grid T={T}", flush=True)
+    Q = np.ones((1, T, d), np.float32)
+    V1 = np.arange(1, d + 1, dtype=np.float32).reshape(1, 1, d)
+    dq, dk, dv = ctx.to_device(Q), ctx.to_device(np.ones_like(V1)), ctx.to_device(V1)
+    do = ctx.to_device(np.full(Q.size + 8, 7.0, np.float32))
+    ctx.sdp_attention(dq, dk, dv, do, 1, T, 1, d, 0.5, False)
+    got = do.download((Q.size + 8,))
+    assert (got[:Q.size].reshape(T, d) == V1[0]).all()
+    assert (got[Q.size:] == 7.0).all()
+
+
 def test_sdp_attention_specials(ctx, orc):
     """-inf scores weigh nothing, a NaN query stays in its row, an infinite value
     in a key that every query of the block may see reaches all of them."""

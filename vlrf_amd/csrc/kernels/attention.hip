@@ -925,7 +925,9 @@ __global__ __launch_bounds__(256, DP <= 64 ? 2 : 1) void attn_f32_mfma_kernel(
     __shared__ float ms[NW][32], ls[NW][32];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: so are the tiles
     const int lq = lane & 31, hh = lane >> 5;
-    const int h = blockIdx.x, q0 = 32 * (int)(gridDim.y - 1 - blockIdx.y);   // the longest causal rows first
+    const int nqb = (T + 31) / 32, qb = (int)(blockIdx.z * gridDim.y + blockIdx.y);   // z: beyond the y limit's blocks
+    if (qb >= nqb) return;
+    const int h = blockIdx.x, q0 = 32 * (nqb - 1 - qb);   // the longest causal rows first
     const float* Kh = K + (size_t)h * ctx * d;
     const float* Vh = V + (size_t)h * ctx * d;
     const int past = ctx - T, qpos = q0 + lq + past;
@@ -938,7 +940,7 @@ __global__ __launch_bounds__(256, DP <= 64 ? 2 : 1) void attn_f32_mfma_kernel(
     };
     float4 qv[NS], kv[NS];
     f32_row<NS, VEC>(qv, tile(Q + (size_t)h * T * d, q0 / 32, T), lq, hh, d);
-    const int first = (w + h + (int)blockIdx.y) % NW;   // the odd tiles fall to another SIMD in each workgroup
+    const int first = (w + h + qb % NW) % NW;   // the odd tiles fall to another SIMD in each workgroup
     f32_row<NS, VEC>(kv, tile(Kh, min(first, ntile - 1), k_limit), lq, hh, d);
     f32_row_zero_past<NS>(qv, hh, d);
 #pragma unroll
@@ -1817,7 +1819,10 @@ int launch_attn_f32_tiled(hipStream_t s, const float* Q, const float* K, const f
     VH_ARG(d_h >= 1 && d_h <= 128, "attn_f32: d_h %d outside [1,128]", d_h);
     VH_ARG(T <= ctx_len || !causal, "attn_f32: causal with T > ctx_len");
     const bool vec = d_h % 4 == 0 && (((uintptr_t)Q | (uintptr_t)K) & 15) == 0;
-    const dim3 grid(n_h, (T + 31) / 32);   // a head's workgroups on one XCD when 8 divides the heads: its K/V in one L2
+    // A head's workgroups on one XCD when 8 divides the heads: its K/V in one L2.
+    // Past 2^20 queries the blocks go on along z (a grid takes 65535 along y).
+    const int nqb = (T + 31) / 32, yb = nqb < 32768 ? nqb : 32768;
+    const dim3 grid(n_h, yb, (nqb + yb - 1) / yb);
     // Scores in powers of 2; a negative scale's sign goes to q, so that the largest score stays the largest.
     const float sl2 = (float)(std::fabs((double)scale) * 1.4426950408889634), qsign = scale < 0.f ? -1.f : 1.f;
 #define VH_AT(DP)                                                                                              \
