@@ -199,6 +199,27 @@ def test_small_m_any_k(ctx, dtype, M, N, K, norm, res):
     assert (np.abs(dy.download((M, N)) - ref) <= bound).all()
 
 
+@pytest.mark.parametrize("M,N,K,norm,res", [
+    (2, 70, 256, True, False), (8, 64, 512, True, True), (9, 63, 2048, True, False), (16, 130, 2304, True, False),
+    (7, 65, 2560, False, True), (16, 40, 4352, True, False), (3, 33, 2304, False, False)])
+def test_small_m_slice_counts(ctx, M, N, K, norm, res):
+    """1, 2, 8, 9, 10 and 17 slices of 256 columns, whose partial sums are added
+    eight slices at a time or one; rows up to eight and more.  x in two bf16
+    pieces is off by at most 2^-16 of itself; with a norm a rounding more."""
+    print(f"[case] small M slices M={M} N={N} K={K} norm={norm} res={res}", flush=True)
+    w, dec = _weight(ctx, 36, f"S{N}x{K}", N, K, V.DT_Q8_0)
+    x = F.normal(36, f"x{M}x{K}", M * K).reshape(M, K)
+    nw = 1 + F.normal(36, f"n{K}", K, 0.1) if norm else None
+    r = F.normal(36, f"r{M}x{N}", M * N).reshape(M, N)
+    dy = ctx.to_device(r)
+    ctx.qlinear(w, ctx.to_device(x), dy, M, norm_w=ctx.to_device(nw) if norm else None, residual=dy if res else None)
+    ref, bound = _small_bound(x, dec, nw)
+    bound = bound * (1 + 2.0 ** 8 / K)   # + 2^-16 of the absolute sum, in units of K eps
+    if res:
+        ref, bound = ref + r, bound + 2.0 ** -23 * (np.abs(ref) + np.abs(r))
+    assert (np.abs(dy.download((M, N)) - ref) <= bound).all()
+
+
 @pytest.mark.parametrize("dtype", [V.DT_Q8_0, V.DT_Q4_0])
 @pytest.mark.parametrize("M,N,K", [(16, 70, 352), (3, 200, 1504)])
 def test_small_m_any_k_swiglu_and_specials(ctx, orc, dtype, M, N, K):

@@ -1703,15 +1703,18 @@ __device__ __forceinline__ void split3(float v, uint32_t& h, uint32_t& m, uint32
     l = __float_as_uint(r - __uint_as_float(m)) & 0xFFFF0000u;
 }
 
+__device__ __forceinline__ float4 select4(bool c, const float4& v, float other) {
+    return make_float4(c ? v.x : other, c ? v.y : other, c ? v.z : other, c ? v.w : other);
+}
+
 // ANY: K any multiple of 32, the last slice with what is left (its missing
 // columns are zeros of x under zero scales), and x in three pieces, so that
 // the products carry all of its 24 bits: those K ran on the f32 vector kernel,
 // whose error against 64 bits (1e-7) two pieces (3e-6) would not keep.
 template <int WT, int NM, int EPI, int NW, bool ANY>
 __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
-    const uint8_t* __restrict__ qa, const __half* __restrict__ da, const uint8_t* __restrict__ qb,
-    const __half* __restrict__ db, int N, int K, int M, const float* __restrict__ x,
-    const float* __restrict__ norm_w, float eps, const float* __restrict__ residual, float* __restrict__ y,
+    const uint8_t* qa, const __half* da, const uint8_t* qb, const __half* db, int N, int K, int M, const float* x,
+    const float* norm_w, float eps, const float* __restrict__ residual, float* __restrict__ y,
     float* __restrict__ P, float* __restrict__ SS, int* __restrict__ tile_ctr) {
     constexpr int CB = WT == VLRF_HIP_DT_Q8_0 ? 256 : 128;   // code bytes of a row per slice
     constexpr int CS = CB + 16;                          // padded LDS row stride
@@ -1749,22 +1752,30 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
                 acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
         }
-        // Activations first (L2, needed first), then the codes and scales (HBM):
-        // loads complete in order, so the staging below waits for x only.
+        // Activations and norm weights first (L2, needed first), then the codes and
+        // scales (HBM): loads complete in order, so the staging below waits for the
+        // first only.  No branch from here to the staged tile (rows and columns past
+        // the end read the last ones and are zeroed): over branches the compiler
+        // moved the code loads behind the staging.
+        const bool kin = !ANY || k0 + sk < K;
+        const int kc = ANY ? min(k0 + sk, K - 8) : k0 + sk;
         float4 a0[NI], a1[NI];
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int sm = (tid >> 5) + 2 * NW * i;
             a0[i] = a1[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (sm < M && (!ANY || k0 + sk < K)) {
-                const float4* xp = reinterpret_cast<const float4*>(x + (size_t)sm * K + k0 + sk);
+            if (i == 0 || 2 * NW * i < M) {   // uniform: up to eight rows load no second eight
+                const float4* xp = reinterpret_cast<const float4*>(x + (size_t)min(sm, M - 1) * K + kc);
                 a0[i] = xp[0];
                 a1[i] = xp[1];
             }
         }
+        const float4* wp = reinterpret_cast<const float4*>((norm_w ? norm_w : x) + kc);
+        const float4 w0 = wp[0], w1 = wp[1];
+        __builtin_amdgcn_sched_barrier(0);
         // Codes: load i of lane l covers row LPR-group i*64/LPR + l/LPR, bytes
         // 16(l % LPR) .. +15 of the row's slice: runs of CB contiguous bytes.
-        uint4 cv[NM][CL];
+        dq_u32x4 cv[NM][CL];
         uint32_t sv[NM];
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
@@ -1775,7 +1786,7 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
                 const int r = min(rbase + i * (64 / LPR) + lane / LPR, N - 1);
                 size_t o = (size_t)k0 * CB / kSmallSlice + 16 * (lane % LPR);
                 if constexpr (ANY) o = o < rowb - 16 ? o : rowb - 16;
-                cv[m][i] = *reinterpret_cast<const uint4*>(q + r * rowb + o);
+                cv[m][i] = *reinterpret_cast<const dq_u32x4*>(q + r * rowb + o);
             }
             const int r = min(rbase + (lane >> 2), N - 1);      // 16 rows x 4 dwords of scales
             if constexpr (ANY) {                                // rows of any number of blocks: 2-byte loads
@@ -1787,20 +1798,17 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
                 sv[m] = *reinterpret_cast<const uint32_t*>(d + (size_t)r * (K / 32) + k0 / 32 + 2 * (lane & 3));
             }
         }
+        __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the staging
+        const float4 g0 = select4(norm_w && kin, w0, 1.f), g1 = select4(norm_w && kin, w1, 1.f);
 #pragma unroll
         for (int it = 0; it < NI; ++it) {
             const int sm = (tid >> 5) + 2 * NW * it;
-            float4 b0 = a0[it], b1 = a1[it];
-            if (sm < M && (!ANY || k0 + sk < K)) {
-                ss[it] += b0.x * b0.x + b0.y * b0.y + b0.z * b0.z + b0.w * b0.w +
-                          b1.x * b1.x + b1.y * b1.y + b1.z * b1.z + b1.w * b1.w;
-                if (norm_w) {
-                    const float4* wp = reinterpret_cast<const float4*>(norm_w + k0 + sk);
-                    const float4 w0 = wp[0], w1 = wp[1];
-                    b0 = make_float4(b0.x * w0.x, b0.y * w0.y, b0.z * w0.z, b0.w * w0.w);
-                    b1 = make_float4(b1.x * w1.x, b1.y * w1.y, b1.z * w1.z, b1.w * w1.w);
-                }
-            }
+            const bool live = sm < M && kin;
+            float4 b0 = select4(live, a0[it], 0.f), b1 = select4(live, a1[it], 0.f);
+            ss[it] += b0.x * b0.x + b0.y * b0.y + b0.z * b0.z + b0.w * b0.w +
+                      b1.x * b1.x + b1.y * b1.y + b1.z * b1.z + b1.w * b1.w;
+            b0 = make_float4(b0.x * g0.x, b0.y * g0.y, b0.z * g0.z, b0.w * g0.w);
+            b1 = make_float4(b1.x * g1.x, b1.y * g1.y, b1.z * g1.z, b1.w * g1.w);
             const float v[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
             uint32_t h[4], l[4];
             const int o = (sk >> 5) * 512 + sm * 32 + (sk & 31);
@@ -1831,7 +1839,7 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
         for (int m = 0; m < NM; ++m) {
 #pragma unroll
             for (int i = 0; i < CL; ++i)
-                *reinterpret_cast<uint4*>(&cs[m][wave][(i * (64 / LPR) + lane / LPR) * CS + 16 * (lane % LPR)]) =
+                *reinterpret_cast<dq_u32x4*>(&cs[m][wave][(i * (64 / LPR) + lane / LPR) * CS + 16 * (lane % LPR)]) =
                     cv[m][i];
             ssc[m][wave][lane] = sv[m];
         }
@@ -1913,37 +1921,50 @@ __global__ __launch_bounds__(64 * NW) void qlinear_small_kernel(
     if (n >= N || 4 * q4 >= M) return;
     // Byte offsets stay below 2^32: the partials are S * NM * N * 64 bytes and
     // the host bounds that (qlinear_small_scratch).
+    // Eight slices' loads of every matrix and of the sums of squares are in flight
+    // at a time, each added in slice order (four of one matrix and one of the sums
+    // before, 12 device-coherent round trips for SwiGLU with a norm over 8 slices;
+    // with the staging's order above, us: SwiGLU 2 x 5632 x 2048 at M = 6 12.8 -> 11.1,
+    // 5632 x 2048 with a norm at M = 16 11.1 -> 9.2, 2048 x 5632 at M = 4 9.4 -> 8.9).
     const uint32_t st = (uint32_t)NM * N * 64;                      // bytes per slice
     const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(P, 0, 0x7fffffff, 0x00020000);
-    float4 o[NM];
+    const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc(SS ? SS : P, 0, 0x7fffffff, 0x00020000);
+    const uint32_t base = (uint32_t)((size_t)n * 64 + 16 * q4), mat = (uint32_t)N * 64;
+    const uint32_t sbase = (uint32_t)(((size_t)blockIdx.x * S * 16 + 4 * q4) * 4);
+    float4 o[NM], ssum = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-    for (int j = 0; j < NM; ++j) {
-        const uint32_t base = (uint32_t)(((size_t)j * N + n) * 64 + 16 * q4);
-        float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-        int sl = 0;
-        for (; sl + 4 <= S; sl += 4) {        // four independent loads in flight, added in slice order
-            float4 v4[4];
+    for (int j = 0; j < NM; ++j) o[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto add = [](float4& t, const float4 v) { t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w; };
+    auto pass = [&](auto n_slices, int sl) {   // slices sl .. sl + B - 1; past the last one it is read again, not added
+        constexpr int B = decltype(n_slices)::value;
+        float4 v4[NM][B], s4[B];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) v4[u] = ld_agent4(prs, base + (uint32_t)(sl + u) * st);
+        for (int u = 0; u < B; ++u) {
+            const uint32_t su = (uint32_t)min(sl + u, S - 1);
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                t.x += v4[u].x; t.y += v4[u].y; t.z += v4[u].z; t.w += v4[u].w;
+            for (int j = 0; j < NM; ++j) v4[j][u] = ld_agent4(prs, base + j * mat + su * st);
+        }
+        if (SS) {
+#pragma unroll
+            for (int u = 0; u < B; ++u) s4[u] = ld_agent4(srs, sbase + 64 * (uint32_t)min(sl + u, S - 1));
+        }
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+            if (sl + u < S) {
+#pragma unroll
+                for (int j = 0; j < NM; ++j) add(o[j], v4[j][u]);
             }
+        if (SS) {
+#pragma unroll
+            for (int u = 0; u < B; ++u)
+                if (sl + u < S) add(ssum, s4[u]);
         }
-        for (; sl < S; ++sl) {
-            const float4 v4 = ld_agent4(prs, base + (uint32_t)sl * st);
-            t.x += v4.x; t.y += v4.y; t.z += v4.z; t.w += v4.w;
-        }
-        o[j] = t;
-    }
+    };
+    int sl = 0;
+    for (; sl + 1 < S; sl += 8) pass(std::integral_constant<int, 8>{}, sl);
+    if (sl < S) pass(std::integral_constant<int, 1>{}, sl);   // one left (256 x 256: all of it)
     float inv[4] = {1.f, 1.f, 1.f, 1.f};
     if (SS) {
-        const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc(SS, 0, 0x7fffffff, 0x00020000);
-        float4 ssum = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int sl = 0; sl < S; ++sl) {
-            const float4 v4 = ld_agent4(srs, (uint32_t)((((size_t)blockIdx.x * S + sl) * 16 + 4 * q4) * 4));
-            ssum.x += v4.x; ssum.y += v4.y; ssum.z += v4.z; ssum.w += v4.w;
-        }
         const float sv[4] = {ssum.x, ssum.y, ssum.z, ssum.w};
 #pragma unroll
         for (int u = 0; u < 4; ++u) inv[u] = 1.f / sqrtf(sv[u] / (float)K + eps);
