@@ -878,8 +878,11 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(
 // Plain 64-bit addresses ran 64.6, these loads 41; eight waves a block 44.6.
 //
 // Weights are exp2(s * sl2 - m * sl2) with one rounding at the difference's
-// size and the scores' sums run in two chains: the error against 64 bits over
-// these shapes is at or below the vector kernel's (3.4e-7 against 4.0e-7 at 777).
+// size, the scores' sums run in four chains and the result is one division: the
+// error against 64 bits is at or below the vector kernel's from 5 x 5 keys on
+// (8.1e-8 against 8.2e-8; 100 x 100 at d 128 2.1e-7 against 2.7e-7, 1000 x 1700 at
+// d 80 4.5e-7 against 7.5e-7).  Two chains and a product with 1 / L: 2.9e-7 at
+// 100 x 100, 36.4 us at 777 x 777 against 37.4.
 //
 // DP: d rounded up to 16, zeros beyond d in both q and K.  VEC: 16-byte loads
 // (d % 4 == 0, aligned bases).  Masked keys weigh 0; as in the reference's
@@ -967,21 +970,21 @@ __global__ __launch_bounds__(256, DP <= 64 ? 2 : 1) void attn_f32_mfma_kernel(
                     float, __builtin_amdgcn_raw_buffer_load_b32(vr, vo[c] + 4 * (8 * (r >> 2) + (r & 3)) * d, 0, 0));
         if (DP > d) f32_row_zero_past<NS>(kv, hh, d);
         __builtin_amdgcn_sched_barrier(0);
-        f32x16 s = {}, s1 = {};   // two chains: half the roundings in a row
+        f32x16 s = {}, s1 = {}, s2 = {}, s3 = {};   // four chains: a quarter of the roundings in a row
 #pragma unroll
         for (int i = 0; i < NS; i += 2) {
             s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].x, qv[i].x, s, 0, 0, 0);
             s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i + 1].x, qv[i + 1].x, s1, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].y, qv[i].y, s, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i + 1].y, qv[i + 1].y, s1, 0, 0, 0);
+            s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].y, qv[i].y, s2, 0, 0, 0);
+            s3 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i + 1].y, qv[i + 1].y, s3, 0, 0, 0);
             s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].z, qv[i].z, s, 0, 0, 0);
             s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i + 1].z, qv[i + 1].z, s1, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].w, qv[i].w, s, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i + 1].w, qv[i + 1].w, s1, 0, 0, 0);
+            s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i].w, qv[i].w, s2, 0, 0, 0);
+            s3 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i + 1].w, qv[i + 1].w, s3, 0, 0, 0);
         }
         f32_row<NS, VEC>(kv, tile(Kh, min(t + NW, ntile - 1), k_limit), lq, hh, d);
         __builtin_amdgcn_sched_barrier(0);
-        s += s1;
+        s = (s + s1) + (s2 + s3);
         // Keys past the query's last one weigh 0: only tiles that reach past the
         // block's first query's last key hold any.
         const bool edge = k0 + 31 > (causal ? min(q0 + past, k_limit - 1) : k_limit - 1);
@@ -1045,13 +1048,12 @@ __global__ __launch_bounds__(256, DP <= 64 ? 2 : 1) void attn_f32_mfma_kernel(
         f[i] = ms[i][q] == kNegInf ? 0.f : __builtin_amdgcn_exp2f(ms[i][q] - M);
         L += f[i] * ls[i][q];
     }
-    const float inv = L > 0.f ? 1.f / L : 0.f;
     float* Oq = O + ((size_t)h * T + q0 + q) * d;
     for (int i = part; i < d; i += TPQ) {
         float x = 0.f;
 #pragma unroll
         for (int j = 0; j < NW; ++j) x += f[j] * os[j][q * OS + i];
-        Oq[i] = x * inv;
+        Oq[i] = L > 0.f ? x / L : x * 0.f;   // one rounding
     }
 }
 
