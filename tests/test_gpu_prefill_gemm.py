@@ -275,6 +275,30 @@ def test_bf16_expansion_swiglu_equals_in_register_decode(ctx, monkeypatch, dtype
     _check_forms(a, b, c)
 
 
+@pytest.mark.parametrize("M,N,K,swiglu", [(233, 2560, 2048, False), (166, 4343, 1280, False), (300, 1024, 4096, False),
+                                          (317, 1100, 1536, True)])
+def test_half_size_tiles_keep_the_bits(ctx, monkeypatch, M, N, K, swiglu):
+    """Half-size tiles over the codes (the default at these shapes) add the same
+    slices of K as the plan's own tiles over the bf16 expansion
+    (VLRF_HIP_PREFILL_DQ=0): the same result to the bit."""
+    print(f"[case] half-size tiles M={M} N={N} K={K} swiglu={swiglu}", flush=True)
+    ws = [_weight(ctx, 30, f"H{i}.{N}x{K}", N, K, V.DT_Q4_0)[0] for i in range(1 + swiglu)]
+    dx = ctx.to_device(F.normal(30, f"hx{M}x{K}", M * K).reshape(M, K))
+    out = []
+    for dq in (None, "0"):
+        if dq is None:
+            monkeypatch.delenv("VLRF_HIP_PREFILL_DQ", raising=False)
+        else:
+            monkeypatch.setenv("VLRF_HIP_PREFILL_DQ", dq)
+        dy = ctx.alloc(M * N * 4)
+        if swiglu:
+            ctx.qlinear_swiglu(ws[0], ws[1], dx, dy, M)
+        else:
+            ctx.qlinear(ws[0], dx, dy, M)
+        out.append(dy.download((M, N)))
+    assert np.array_equal(*out)
+
+
 def test_bf16_expansion_is_counted_in_the_weight_bytes(ctx):
     """vlrf_hip_weight_bytes: the packed codes and scales, plus 2 bytes per
     weight once a GEMM of more than 128 rows has made the bf16 expansion."""

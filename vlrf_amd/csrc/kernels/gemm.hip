@@ -1459,13 +1459,20 @@ KSplit split_k(long tiles, int K, int cus, int least = 8) {
 
 // Where the plan's tiles and slices fill at most half of the CUs (small N or
 // short K), tiles of half the columns and, above 128 rows, half the rows, four
-// waves and three stages of A each, in at most 24 slices of at least 4 steps:
-// more and shorter workgroups.  Two slices of up to 16 steps do not pay for their
-// reduction, nor small tiles for their operands beyond 2.5 rounds.  us, the
-// plan's tiles / these: 1236 x 1344, M = 38, 15.5 / 11.0; 345 x 1216, M = 324, 17.0 /
-// 12.1; 2270 x 1216, M = 434, 22.9 / 15.7; 1.1B QKV and O at M = 233 21.7 / 17.9, 20.0 /
-// 16.6; SwiGLU 383 x 1152, M = 202, 21.4 / 12.3.  At more than half a round: 8B QKV,
-// M = 100, 25.0 / 25.3; 8B down, M = 400, 90 / 111.
+// waves and three stages of A each: more workgroups.  Small tiles do not pay for
+// their operands beyond 2.5 rounds.
+//
+// A result's bits depend on the slices alone, so slices of the plan that are
+// alike, of whole pairs of steps, are kept: the tiles then change no result,
+// and both forms above 128 rows agree to the bit whichever tiles each takes.  us, the
+// plan's tiles / these / these in slices of their own: 1.1B QKV at M = 233 20.3 /
+// 18.9 / 17.2, O 19.1 / 16.0 / 16.0; 1024 x 1024, M = 256, 15.8 / 13.0 / 12.2;
+// 397 x 4096, M = 108, 17.1 / 15.0 / 16.5; 4343 x 1280, M = 166, 19.9 / 18.8 / 14.2.
+// Any other K takes at most 24 slices of at least 4 steps, but not two slices of
+// up to 16 steps, which do not pay for their reduction: 1236 x 1344, M = 38, 15.5 ->
+// 11.0; 345 x 1216, M = 324, 17.0 -> 12.1; 2270 x 1216, M = 434, 22.9 -> 15.7; SwiGLU
+// 383 x 1152, M = 202, 21.4 -> 12.3.  At more than half a round: 8B QKV, M = 100,
+// 25.0 -> 25.3; 8B down, M = 400, 90 -> 111.
 using FewTile64 = BTile<64, 128, 2, 2>;
 using FewTile128 = BTile<128, 64, 4, 1>;
 
@@ -1474,8 +1481,11 @@ KSplit few_split(const DevWeight& w, int M, bool swiglu, const KSplit& own, long
     const int bm = M <= 64 ? FewTile64::BM : FewTile128::BM, bn = (M <= 64 ? FewTile64::BN : FewTile128::BN) / (swiglu ? 2 : 1);
     const long few = (long)((M + bm - 1) / bm) * ((w.N + bn - 1) / bn);
     if (2 * few > 5L * cus) return own;
-    KSplit ks = split_k(few, w.K, cus < 24 * few ? cus : (int)(24 * few), 4);
-    if (ks.S == 2 && w.K <= 16 * 64) ks = {1, w.K};
+    KSplit ks = own;
+    if (own.S == 1 || w.K % (128 * own.S)) {
+        ks = split_k(few, w.K, cus < 24 * few ? cus : (int)(24 * few), 4);
+        if (ks.S == 2 && w.K <= 16 * 64) ks = {1, w.K};
+    }
     ks.few = true;
     return ks;
 }
