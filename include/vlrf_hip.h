@@ -175,6 +175,13 @@ int vlrf_hip_qlinear(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t w, const float* x, fl
 int vlrf_hip_qlinear_swiglu(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t wg, vlrf_hip_weight_t wu,
                             const float* x, float* h, int M, const float* norm_w, float eps);
 
+/* How vlrf_hip_qlinear (swiglu: _swiglu) splits the K of a call of M > 16 rows: out =
+ * {slices, columns of a slice (the last one: what is left), 1 on half-size tiles
+ * over the codes, bytes of partial sums}; {1, K, 0, 0} where K stays whole and for
+ * what those calls refuse.  Which slices there are decides the bits of a result.
+ * No device needed (256 CUs are assumed without one). */
+int vlrf_hip_qgemm_plan(int dtype, int M, int N, int K, int swiglu, int64_t out[4]);
+
 /* ============================================================================
  * Edge ops
  * ========================================================================== */

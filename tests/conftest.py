@@ -36,3 +36,12 @@ def rel_err(a, b):
     b = np.asarray(b, np.float64)
     den = np.max(np.abs(b))
     return float(np.max(np.abs(a - b)) / den) if den > 0 else float(np.max(np.abs(a - b)))
+
+
+def gemm_plan(dtype, M, N, K, swiglu=False):
+    """(slices of K, columns of one, half-size tiles, bytes of partial sums) of a GEMM of M rows."""
+    import ctypes as C
+    import vlrf_amd as V
+    out = (C.c_int64 * 4)()
+    V.check(V.lib().vlrf_hip_qgemm_plan(dtype, M, N, K, int(swiglu), out))
+    return out[0], out[1], bool(out[2]), out[3]

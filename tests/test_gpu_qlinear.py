@@ -164,6 +164,23 @@ def test_qlinear_rejects_bad_shapes(ctx):
         ctx.qlinear(w, x, x, 1)                             # x aliasing y
 
 
+@pytest.mark.parametrize("dtype,K", [(V.DT_Q8_0, 32), (V.DT_Q4_0, 32), (V.DT_Q8_0, 96), (V.DT_F32, 32), (V.DT_F32, 64)])
+def test_qlinear_rejects_bad_k_above_128_rows(ctx, dtype, K):
+    """K below a step of 64 (no step to split) or off it, and f32 weights: an
+    argument error from both forms, and the context goes on."""
+    M, N = 129, 64
+    print(f"[case] refused K={K} dtype={dtype}", flush=True)
+    wf = F.normal(11, f"Wk{K}", N * K, 0.02)
+    w = V.QuantWeight(ctx, F.quantize(wf, dtype) if dtype != V.DT_F32 else wf, dtype, N, K)
+    x, y = ctx.alloc(M * K * 4), ctx.alloc(M * N * 4)
+    with pytest.raises(V.HipError):
+        ctx.qlinear(w, x, y, M)
+    with pytest.raises(V.HipError):
+        ctx.qlinear_swiglu(w, w, x, y, M)
+    ctx.qlinear(w, x, y, 16)
+    ctx.sync()
+
+
 def _small_bound(x, dec, nw, eps=1e-5):
     """(y, bound) in 64 bits: f32 sums of K products, exact in pieces, are off by
     at most (K + 60) eps of the absolute sum; a fused norm adds (K / 2 + 10) eps."""

@@ -699,6 +699,16 @@ int vlrf_hip_qlinear_swiglu(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t wg, vlrf_hip_w
     return launch_qgemm_swiglu(ctx->stream, wg->w, wu->w, a, M, h, false, part);
 }
 
+int vlrf_hip_qgemm_plan(int dtype, int M, int N, int K, int swiglu, int64_t out[4]) {
+    VH_ARG(out && M >= 1 && N >= 1 && K >= 1, "qgemm_plan: bad arguments");
+    DevWeight w;
+    w.dtype = dtype;
+    w.N = N;
+    w.K = K;
+    qgemm_plan(w, M, swiglu != 0, out);
+    return VLRF_HIP_OK;
+}
+
 // ---- the engine's remaining per-op backend calls --------------------------------------
 int vlrf_hip_gemm_f32(vlrf_hip_ctx_t ctx, const float* A, const float* B, float* C, int M, int N, int K,
                       int lda, int ldb, int ldc, float alpha, float beta, int transA, int transB) {

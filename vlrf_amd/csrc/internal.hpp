@@ -195,6 +195,7 @@ int launch_qgemm(hipStream_t s, const DevWeight& w, const uint16_t* a, int M, co
 int launch_qgemm_swiglu(hipStream_t s, const DevWeight& wg, const DevWeight& wu, const uint16_t* a,
                         int M, void* h, bool h_bf16, float* part = nullptr);
 size_t qgemm_part_bytes(const DevWeight& w, int M, bool swiglu);
+void qgemm_plan(const DevWeight& w, int M, bool swiglu, int64_t out[4]);   // vlrf_hip_qgemm_plan
 // Small M (2..16) on the matrix cores with f32-class accuracy (x split into
 // bf16 hi + lo): y = x.W0^T (+ residual), or silu(x.W0^T) * (x.W1^T) when w1
 // is given, in one launch.  Per-slice partial sums go to scratch

@@ -1438,7 +1438,7 @@ struct KSplit {
 };
 
 // As many slices as fit one round of the CUs beside each other (tiles output
-// tiles), of at least `least` steps: a number down to 3/4 of that which divides the
+// tiles; K of at least one step), of at least `least` steps: a number down to 3/4 of that which divides the
 // steps, if there is one (8B QKV at M = 100, 48 tiles of 64 steps: 4 slices 23.9
 // us, 5 uneven ones 24.4), else that many, as even as whole steps allow.  (us at
 // Q8_0, slices that had to divide K / 128 or none -> these: 4123 x 10944, M = 105,
@@ -2121,11 +2121,25 @@ bool weight_expand_bf16(hipStream_t s, const DevWeight& w) {
 // needs (0 when it runs unsplit or on another kernel).
 static bool dq_split_path(const DevWeight& w, int M) { return M >= 17 && M <= 128 && dqgemm_supported(w); }
 
+// K whole wherever no split applies, and for what check_qgemm refuses: callers
+// size their scratch with this before the check.
+static KSplit gemm_split(const DevWeight& w, int M, bool swiglu) {
+    if ((w.dtype != VLRF_HIP_DT_Q8_0 && w.dtype != VLRF_HIP_DT_Q4_0) || w.K < kBK || w.K % kBK) return {1, w.K};
+    if (M > 128) return big_split(w, M, swiglu, lds_cus());
+    return dq_split_path(w, M) ? mid_split(w, M, swiglu, lds_cus()) : KSplit{1, w.K};
+}
+
 size_t qgemm_part_bytes(const DevWeight& w, int M, bool swiglu) {
-    int S = 1;
-    if (M > 128) S = big_split(w, M, swiglu, lds_cus()).S;
-    else if (dq_split_path(w, M)) S = mid_split(w, M, swiglu, lds_cus()).S;
+    const int S = gemm_split(w, M, swiglu).S;
     return S > 1 ? (size_t)S * M * w.N * (swiglu ? 2 : 1) * sizeof(float) : 0;
+}
+
+void qgemm_plan(const DevWeight& w, int M, bool swiglu, int64_t out[4]) {
+    const KSplit ks = gemm_split(w, M, swiglu);
+    out[0] = ks.S;
+    out[1] = ks.kl;
+    out[2] = ks.few;
+    out[3] = (int64_t)qgemm_part_bytes(w, M, swiglu);
 }
 
 int launch_qgemm(hipStream_t s, const DevWeight& w, const uint16_t* a, int M, const float* residual,
@@ -2135,7 +2149,7 @@ int launch_qgemm(hipStream_t s, const DevWeight& w, const uint16_t* a, int M, co
     VH_ARG(a && y, "qgemm: null operand");
     if (M > 128) {
         weight_expand_bf16(s, w);
-        const KSplit ks = part || !qgemm_part_bytes(w, M, false) ? big_split(w, M, false, lds_cus()) : KSplit{1, w.K};
+        const KSplit ks = part || !qgemm_part_bytes(w, M, false) ? gemm_split(w, M, false) : KSplit{1, w.K};
         if (ks.few) {
             if (residual) launch_dq_split<1>(s, a, w, nullptr, M, ks, residual, y, part);
             else launch_dq_split<0>(s, a, w, nullptr, M, ks, nullptr, y, part);
@@ -2154,7 +2168,7 @@ int launch_qgemm(hipStream_t s, const DevWeight& w, const uint16_t* a, int M, co
             else launch_lds_plan<0>(s, p, a, w, nullptr, M, nullptr, y);
         }
     } else if (dq_split_path(w, M) && (part || qgemm_part_bytes(w, M, false) == 0)) {
-        const KSplit ks = mid_split(w, M, false, lds_cus());
+        const KSplit ks = gemm_split(w, M, false);
         if (residual) launch_dq_split<1>(s, a, w, nullptr, M, ks, residual, y, part);
         else launch_dq_split<0>(s, a, w, nullptr, M, ks, nullptr, y, part);
     } else {
@@ -2181,7 +2195,7 @@ int launch_qgemm_swiglu(hipStream_t s, const DevWeight& wg, const DevWeight& wu,
             (void)hipFree(wg.bf);   // both or neither (no free while capturing)
             wg.bf = nullptr;
         }
-        const KSplit ks = part || !qgemm_part_bytes(wg, M, true) ? big_split(wg, M, true, lds_cus()) : KSplit{1, wg.K};
+        const KSplit ks = part || !qgemm_part_bytes(wg, M, true) ? gemm_split(wg, M, true) : KSplit{1, wg.K};
         if (ks.few) {
             if (h_bf16) launch_dq_split<2>(s, a, wg, &wu, M, ks, nullptr, h, part);
             else launch_dq_split<3>(s, a, wg, &wu, M, ks, nullptr, h, part);
@@ -2200,7 +2214,7 @@ int launch_qgemm_swiglu(hipStream_t s, const DevWeight& wg, const DevWeight& wu,
             else launch_lds_plan<3>(s, p, a, wg, &wu, M, nullptr, h);
         }
     } else if (dq_split_path(wg, M) && (part || qgemm_part_bytes(wg, M, true) == 0)) {
-        const KSplit ks = mid_split(wg, M, true, lds_cus());
+        const KSplit ks = gemm_split(wg, M, true);
         if (h_bf16) launch_dq_split<2>(s, a, wg, &wu, M, ks, nullptr, h, part);
         else launch_dq_split<3>(s, a, wg, &wu, M, ks, nullptr, h, part);
     } else {
