@@ -74,6 +74,9 @@ int   vlrf_hip_d2d(vlrf_hip_ctx_t ctx, void* dst, const void* src, size_t bytes)
 /* Event timing on the context stream: records start/stop around queued work. */
 int   vlrf_hip_timer_start(vlrf_hip_ctx_t ctx);
 int   vlrf_hip_timer_stop(vlrf_hip_ctx_t ctx, float* ms);  /* waits for the stop event */
+/* out = {bytes of the context's scratch buffer, bytes of outgrown ones that it keeps
+ * because launches captured into a graph address them}; both go with the context. */
+int   vlrf_hip_scratch_bytes(vlrf_hip_ctx_t ctx, size_t out[2]);
 
 /* ============================================================================
  * Attention

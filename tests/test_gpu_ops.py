@@ -119,6 +119,52 @@ def test_gemm_f32_under_graph_capture():
     hip.hipGraphDestroy(g)
 
 
+def test_captured_calls_outlive_scratch_growth():
+    """A captured K-split GEMM keeps the scratch address it recorded: eager calls
+    that outgrow the buffer (an f32 GEMM, a small-M linear, twice) leave it in
+    place, and every replay gives the eager result.  Replayed only once the
+    context says that it kept the old buffer."""
+    import ctypes as C
+    from test_gpu_prefill_gemm import _hip
+    hip, ctx = _hip(), V.Context(0)
+
+    def held():
+        out = (C.c_size_t * 2)()
+        V.check(V.lib().vlrf_hip_scratch_bytes(ctx.h, out))
+        return out[0], out[1]
+
+    M, N, K = 64, 512, 1024
+    w = V.QuantWeight(ctx, F.quantize(F.normal(69, "w", N * K, 0.02), V.DT_Q8_0), V.DT_Q8_0, N, K)
+    dx, dy = ctx.to_device(F.normal(69, "x", M * K)), ctx.alloc(M * N * 4)
+    ctx.qlinear(w, dx, dy, M)
+    eager = dy.download((M, N))
+    s, g, ge = C.c_void_p(ctx.stream()), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(s, 2) == 0
+    rc = V.lib().vlrf_hip_qlinear(ctx.h, w.h, dx.ptr, dy.ptr, M, None, C.c_float(0.0), None)
+    assert hip.hipStreamEndCapture(s, C.byref(g)) == 0 and rc == 0
+    assert hip.hipGraphInstantiate(C.byref(ge), g, None, None, 0) == 0
+    small, kept = held()
+    assert small > 0 and kept == 0
+    m, n, k = 64, 512, 16384                                            # splits K: m n 4 bytes a slice
+    A, B, Cb = ctx.to_device(F.normal(69, "A", m * k)), ctx.to_device(F.normal(69, "B", n * k)), ctx.alloc(m * n * 4)
+    n2, k2 = 9000, 4128                                                 # any-K small-M: more partials than that
+    w2 = V.QuantWeight(ctx, F.quantize(F.normal(69, "w2", n2 * k2, 0.02), V.DT_Q8_0), V.DT_Q8_0, n2, k2)
+    x2, y2 = ctx.to_device(F.normal(69, "x2", 16 * k2)), ctx.alloc(16 * n2 * 4)
+    for grow in (lambda: ctx.gemm_f32(A, B, Cb, m, n, k, trans_b=True), lambda: ctx.qlinear(w2, x2, y2, 16)):
+        before = held()[0]
+        grow()
+        ctx.sync()
+        assert held()[0] > before and held()[1] == small                # the captured one, and no other
+        for _ in range(3):
+            dy.zero()
+            grow()
+            assert hip.hipGraphLaunch(ge, s) == 0
+            ctx.sync()
+            assert np.array_equal(dy.download((M, N)), eager)
+    hip.hipGraphExecDestroy(ge)
+    hip.hipGraphDestroy(g)
+
+
 def test_gemm_f32_rejects_bad_shapes(ctx):
     a = ctx.alloc(64)
     with pytest.raises(V.HipError):

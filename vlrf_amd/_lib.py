@@ -56,6 +56,7 @@ _SIGS = {
     "vlrf_hip_weight_upload": (i32, [vp, vp, i32, i32, i32, C.POINTER(vp)]),
     "vlrf_hip_weight_free": (None, [vp]),
     "vlrf_hip_qgemm_plan": (i32, [i32, i32, i32, i32, i32, C.POINTER(C.c_int64)]),
+    "vlrf_hip_scratch_bytes": (i32, [vp, C.POINTER(sz)]),
     "vlrf_hip_weight_bytes": (sz, [vp]),
     "vlrf_hip_qlinear": (i32, [vp, vp, vp, vp, i32, vp, f32, vp]),
     "vlrf_hip_qlinear_swiglu": (i32, [vp, vp, vp, vp, vp, i32, vp, f32]),

@@ -5,6 +5,7 @@
 #include "internal.hpp"
 #include "runtime.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
@@ -146,43 +147,61 @@ int vlrf_hip_ctx::rope_tables(int max_seq, int d_head, float theta, const float*
     return VLRF_HIP_OK;
 }
 
+static bool stream_capturing(hipStream_t s) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 int vlrf_hip_ctx::scratch(size_t bytes, float** out) {
+    const bool capturing = stream_capturing(stream);
     if (bytes > scratch_bytes) {
         // Growing synchronises and allocates, which a stream under graph
         // capture must not record.
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-            (void)hipGetLastError();
+        if (capturing) {
             set_error("scratch: the call needs %zu bytes of context scratch (%zu held) while the stream is being "
                       "captured; make the same call once before capturing", bytes, scratch_bytes);
             return VLRF_HIP_ERR_ARG;
         }
-        if (scratch_buf) {
+        size_t size = bytes;
+        if (scratch_captured) {   // the old buffer stays: a graph's replays use it
+            if (n_kept == kMaxKept) {
+                set_error("scratch: %d outgrown buffers are kept for captured graphs", n_kept);
+                return VLRF_HIP_ERR_NOMEM;
+            }
+            size = std::max(bytes, 2 * scratch_bytes);
+        } else if (scratch_buf) {
             VH_CHECK(hipStreamSynchronize(stream));
             (void)hipFree(scratch_buf);
             scratch_buf = nullptr;
             scratch_bytes = 0;
         }
-        if (hipMalloc(&scratch_buf, bytes) != hipSuccess) {
-            set_error("scratch: hipMalloc(%zu) failed", bytes);
+        void* grown = nullptr;
+        if (hipMalloc(&grown, size) != hipSuccess && (size == bytes || hipMalloc(&grown, size = bytes) != hipSuccess)) {
+            (void)hipGetLastError();
+            set_error("scratch: hipMalloc(%zu) failed", size);
             return VLRF_HIP_ERR_NOMEM;
         }
-        scratch_bytes = bytes;
+        (void)hipGetLastError();
+        if (scratch_captured) {
+            kept[n_kept++] = scratch_buf;
+            kept_bytes += scratch_bytes;
+        }
+        scratch_buf = grown;
+        scratch_bytes = size;
+        scratch_captured = false;
     }
+    scratch_captured |= capturing;
     *out = static_cast<float*>(scratch_buf);
     return VLRF_HIP_OK;
 }
 
 float* vlrf_hip_ctx::try_scratch(size_t bytes) {
     float* p = nullptr;
-    if (!bytes) return nullptr;
-    // Not under capture: a captured launch would keep the address of a buffer
-    // that a later call may regrow.
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
+    // Not under capture: the callers ran without the shared buffer before, so a
+    // graph of theirs may be replayed beside the context's own work.
+    if (!bytes || stream_capturing(stream)) return nullptr;
     if (scratch(bytes, &p) != VLRF_HIP_OK) {
         (void)hipGetLastError();   // the caller goes on: no error is left for its launch check
         return nullptr;
@@ -198,6 +217,7 @@ vlrf_hip_ctx::~vlrf_hip_ctx() {
         (void)hipFree(t.sin_t);
     }
     if (scratch_buf) (void)hipFree(scratch_buf);
+    for (int i = 0; i < n_kept; ++i) (void)hipFree(kept[i]);
     if (small_tile_ctr) (void)hipFree(small_tile_ctr);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
@@ -403,6 +423,14 @@ int vlrf_hip_timer_stop(vlrf_hip_ctx_t ctx, float* ms) {
     VH_CHECK(hipEventRecord(ctx->ev1, ctx->stream));
     VH_CHECK(hipEventSynchronize(ctx->ev1));
     VH_CHECK(hipEventElapsedTime(ms, ctx->ev0, ctx->ev1));
+    return VLRF_HIP_OK;
+}
+
+int vlrf_hip_scratch_bytes(vlrf_hip_ctx_t ctx, size_t out[2]) {
+    VH_CTX(ctx);
+    VH_ARG(out != nullptr, "scratch_bytes: null output");
+    out[0] = ctx->scratch_bytes;
+    out[1] = ctx->kept_bytes;
     return VLRF_HIP_OK;
 }
 
@@ -620,10 +648,7 @@ static int gemm_scratch(Ctx* ctx, int K, size_t a_bytes, size_t p_bytes, float**
         return VLRF_HIP_OK;
     }
     (void)hipGetLastError();
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    const bool capturing = hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
-    (void)hipGetLastError();
-    return p_bytes && (K % 128 || !capturing) ? ctx->scratch(a_bytes, a) : rc;
+    return p_bytes && (K % 128 || !stream_capturing(ctx->stream)) ? ctx->scratch(a_bytes, a) : rc;
 }
 
 // Scratch of the small-M kernel (2 <= M <= 16); null: the call runs on the vector
