@@ -164,7 +164,9 @@ size_t vlrf_hip_weight_bytes(vlrf_hip_weight_t w);   /* device bytes of the pack
  * decoded weights are rounded to bf16, accumulation is f32; it takes Q8_0 or
  * Q4_0 weights with K % 64 == 0 and uses the context's scratch buffer.
  * Graph capture of the stream: the scratch buffer cannot grow while the
- * stream is captured (VLRF_HIP_ERR_ARG: make the same call once first), and a
+ * stream is captured.  A call that needs more is VLRF_HIP_ERR_ARG (make the
+ * same call once first), except that M > 16 runs with K whole, slower, where the
+ * buffer holds its rows but not its partial sums (vlrf_hip_qgemm_plan).  A
  * weight's bf16 expansion is not made then (the GEMM decodes the blocks in its
  * tiles instead, same 1e-2 class). */
 int vlrf_hip_qlinear(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t w, const float* x, float* y, int M,

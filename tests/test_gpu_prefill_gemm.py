@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import vlrf_amd as V
-from conftest import rel_err
+from conftest import gemm_plan, rel_err
 from vlrf_amd import _lib
 from vlrf_amd import formats as F
 
@@ -384,3 +384,40 @@ def test_prefill_gemm_under_graph_capture(orc, dtype, M):
     ctx.qlinear(w1, dx2, y3, M2)                               # eagerly it runs
     ctx.sync()
     assert rel_err(y3.download((M2, N))[:M], ref) <= TOL
+
+
+@pytest.mark.parametrize("M,N,K,swiglu", [(128, 2048, 5504, False), (300, 1024, 4096, False), (100, 600, 2048, True)])
+def test_captured_gemm_with_scratch_for_its_rows_only(M, N, K, swiglu):
+    """Captured when the context scratch holds the call's bf16 rows but not its
+    partial sums: recorded with K whole, not refused; every replay is the eager
+    result up to the order of the f32 sums."""
+    import ctypes as C
+    hip, ctx = _hip(), V.Context(0)
+    print(f"[case] capture, scratch for the rows M={M} N={N} K={K} swiglu={swiglu}", flush=True)
+    ws = [_weight(ctx, 32, f"c{i}", N, K, V.DT_Q8_0)[0] for i in range(1 + swiglu)]
+    one, _ = _weight(ctx, 32, "one", 1, K, V.DT_Q8_0)
+    dx, y, e = ctx.to_device(F.normal(32, "x", M * K).reshape(M, K)), ctx.alloc(M * N * 4), ctx.alloc(M * N * 4)
+    S, _, _, part = gemm_plan(V.DT_Q8_0, M, N, K, swiglu)
+    ctx.qlinear(one, dx, y, M)                                 # the same rows, one column
+    held = (C.c_size_t * 2)()
+    V.check(V.lib().vlrf_hip_scratch_bytes(ctx.h, held))
+    assert S > 1 and 2 * M * K <= held[0] < 2 * M * K + part
+
+    def call(out):
+        if swiglu:
+            return V.lib().vlrf_hip_qlinear_swiglu(ctx.h, ws[0].h, ws[1].h, dx.ptr, out.ptr, M, None, C.c_float(0.0))
+        return V.lib().vlrf_hip_qlinear(ctx.h, ws[0].h, dx.ptr, out.ptr, M, None, C.c_float(0.0), None)
+
+    s, g, ge = C.c_void_p(ctx.stream()), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(s, 2) == 0
+    rc = call(y)
+    assert hip.hipStreamEndCapture(s, C.byref(g)) == 0 and rc == 0, V.lib().vlrf_hip_last_error()
+    assert hip.hipGraphInstantiate(C.byref(ge), g, None, None, 0) == 0
+    for _ in range(3):
+        y.zero()
+        V.check(call(e))                                       # eager, split: grows the scratch the first time
+        assert hip.hipGraphLaunch(ge, s) == 0
+        ctx.sync()
+        assert rel_err(y.download((M, N)), e.download((M, N))) <= 2e-5
+    hip.hipGraphExecDestroy(ge)
+    hip.hipGraphDestroy(g)

@@ -637,18 +637,14 @@ size_t vlrf_hip_weight_bytes(vlrf_hip_weight_t w) {
 }  // extern "C"
 
 // Scratch of a GEMM of M > 16 rows: the bf16 rows, then the K-split partial sums;
-// where both together cannot be had, the rows alone (K then stays whole).  Under
-// capture that holds for K off the multiples of 128 only, whose calls need no
-// partial sums; the others are refused there until the scratch has grown.
-static int gemm_scratch(Ctx* ctx, int K, size_t a_bytes, size_t p_bytes, float** a, float** part) {
+// where both together cannot be had (no memory, or a stream under capture that may
+// not grow the buffer), the rows alone: K then stays whole.
+static int gemm_scratch(Ctx* ctx, size_t a_bytes, size_t p_bytes, float** a, float** part) {
     *part = nullptr;
     int rc = ctx->scratch(a_bytes + p_bytes, a);
-    if (!rc) {
-        if (p_bytes) *part = reinterpret_cast<float*>(reinterpret_cast<char*>(*a) + a_bytes);
-        return VLRF_HIP_OK;
-    }
-    (void)hipGetLastError();
-    return p_bytes && (K % 128 || !stream_capturing(ctx->stream)) ? ctx->scratch(a_bytes, a) : rc;
+    if (rc) return p_bytes ? ctx->scratch(a_bytes, a) : rc;
+    if (p_bytes) *part = reinterpret_cast<float*>(reinterpret_cast<char*>(*a) + a_bytes);
+    return VLRF_HIP_OK;
 }
 
 // Scratch of the small-M kernel (2 <= M <= 16); null: the call runs on the vector
@@ -690,7 +686,7 @@ int vlrf_hip_qlinear(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t w, const float* x, fl
     const size_t a_bytes = ((size_t)M * w->w.K * sizeof(uint16_t) + 255) & ~(size_t)255;
     const size_t p_bytes = qgemm_part_bytes(w->w, M, false);
     float *scratch = nullptr, *part = nullptr;
-    int rc = gemm_scratch(ctx, w->w.K, a_bytes, p_bytes, &scratch, &part);
+    int rc = gemm_scratch(ctx, a_bytes, p_bytes, &scratch, &part);
     if (rc) return rc;
     uint16_t* a = reinterpret_cast<uint16_t*>(scratch);
     rc = launch_rows_to_bf16(ctx->stream, x, norm_w, a, M, w->w.K, eps);
@@ -716,7 +712,7 @@ int vlrf_hip_qlinear_swiglu(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t wg, vlrf_hip_w
     const size_t a_bytes = ((size_t)M * wg->w.K * sizeof(uint16_t) + 255) & ~(size_t)255;
     const size_t p_bytes = qgemm_part_bytes(wg->w, M, true);
     float *scratch = nullptr, *part = nullptr;
-    int rc = gemm_scratch(ctx, wg->w.K, a_bytes, p_bytes, &scratch, &part);
+    int rc = gemm_scratch(ctx, a_bytes, p_bytes, &scratch, &part);
     if (rc) return rc;
     uint16_t* a = reinterpret_cast<uint16_t*>(scratch);
     rc = launch_rows_to_bf16(ctx->stream, x, norm_w, a, M, wg->w.K, eps);
