@@ -202,20 +202,68 @@ def test_swiglu_uneven_k_slices(ctx, monkeypatch, M, Fd, K):
     _check_forms(a, b, c)
 
 
+@pytest.mark.parametrize("dtype", [V.DT_Q8_0, V.DT_Q4_0])
+# slices of 9 steps and a last one of 5 (128 x 128 tiles), 2 (64 x 256), 7, of 16 and 15 (256 rows)
+@pytest.mark.parametrize("M,N,K,res", [(105, 2100, 5504, True), (50, 4500, 4160, False), (300, 2051, 2752, True),
+                                       (700, 4120, 1984, False)])
+def test_gemm_uneven_k_slices_on_whole_tiles(ctx, monkeypatch, dtype, M, N, K, res):
+    """A shorter last slice on the plan's own tiles (the shapes above take the
+    half-size ones): above 128 rows over the expansion and over the codes."""
+    print(f"[case] uneven K slices, whole tiles dtype={dtype} M={M} N={N} K={K} res={res}", flush=True)
+    S, kl, few, _ = gemm_plan(dtype, M, N, K)
+    assert S > 1 and K % kl and not few
+    x = F.normal(28, f"ux{M}x{K}", M * K).reshape(M, K)
+    r = F.normal(28, f"ur{M}x{N}", M * N).reshape(M, N)
+    dx, dec = ctx.to_device(x), []
+
+    def run():
+        w, d = _weight(ctx, 28, f"U{N}x{K}", N, K, dtype)
+        dec.append(d)
+        dy = ctx.to_device(r) if res else ctx.alloc(M * N * 4)
+        ctx.qlinear(w, dx, dy, M, residual=dy if res else None)
+        return dy.download((M, N))
+
+    a, b, c = _all_forms(monkeypatch, run)
+    _check_forms(a, b, c)
+    xb, wb = (_bf16(t).astype(np.float64) for t in (x, dec[0]))
+    ref = xb @ wb.T + (r if res else 0)
+    bound = (K + 40) * 2.0 ** -24 * (np.abs(xb) @ np.abs(wb).T + (np.abs(r) if res else 0))
+    assert (np.abs(a - ref) <= bound).all()
+
+
+# last slices of 9, 1 and 7 steps
+@pytest.mark.parametrize("M,Fd,K", [(128, 2048, 5504), (20, 773, 10432), (300, 2051, 2752)])
+def test_swiglu_uneven_k_slices_on_whole_tiles(ctx, monkeypatch, M, Fd, K):
+    print(f"[case] uneven K slices swiglu, whole tiles M={M} F={Fd} K={K}", flush=True)
+    S, kl, few, _ = gemm_plan(V.DT_Q4_0, M, Fd, K, True)
+    assert S > 1 and K % kl and not few
+    dx = ctx.to_device(F.normal(29, f"vx{M}x{K}", M * K).reshape(M, K))
+
+    def run():
+        wg, _ = _weight(ctx, 29, f"VG{Fd}x{K}", Fd, K, V.DT_Q4_0)
+        wu, _ = _weight(ctx, 29, f"VU{Fd}x{K}", Fd, K, V.DT_Q4_0)
+        dh = ctx.alloc(M * Fd * 4)
+        ctx.qlinear_swiglu(wg, wu, dx, dh, M)
+        return dh.download((M, Fd))
+
+    _check_forms(*_all_forms(monkeypatch, run))
+
+
 def _check_forms(a, b, c):
-    """Expansion and in-LDS forms identical bit for bit; the in-register form
-    identical too, except where the GEMM's few tiles make the two others
-    split K into slices (300 x 4096 x 2048), which it does not: there it
+    """The default and the in-LDS form identical bit for bit (at shapes on
+    half-size tiles both are that one kernel: test_half_size_tiles_keep_the_bits
+    compares it with the expansion); the in-register form identical too, except
+    where the two others split K into slices, which it does not: there it
     differs by the f32 summation order only."""
     assert np.array_equal(a, b)
     assert np.array_equal(a, c) or rel_err(a, c) <= 2e-5, rel_err(a, c)
 
 
 def _all_forms(monkeypatch, run):
-    """run() with the weights' bf16 expansion (the default for M > 128), with
-    VLRF_HIP_PREFILL_BF16=0 (Q8_0 with K % 128 == 0: codes decoded into LDS
-    tiles, once per workgroup; otherwise in registers) and with
-    VLRF_HIP_PREFILL_DQ=0 as well (codes decoded in registers)."""
+    """run() as it comes (above 128 rows over the weights' bf16 expansion, but
+    half-size tiles over the codes), with VLRF_HIP_PREFILL_BF16=0 (codes decoded
+    into LDS tiles, once per workgroup) and with VLRF_HIP_PREFILL_DQ=0 as well
+    (codes decoded in registers, K whole)."""
     monkeypatch.delenv("VLRF_HIP_PREFILL_BF16", raising=False)
     monkeypatch.delenv("VLRF_HIP_PREFILL_DQ", raising=False)
     a = run()
@@ -276,12 +324,15 @@ def test_bf16_expansion_swiglu_equals_in_register_decode(ctx, monkeypatch, dtype
 
 
 @pytest.mark.parametrize("M,N,K,swiglu", [(233, 2560, 2048, False), (166, 4343, 1280, False), (300, 1024, 4096, False),
-                                          (317, 1100, 1536, True)])
+                                          (317, 1100, 1536, True),                            # the plan's slices
+                                          (1000, 1024, 512, False), (257, 1000, 256, False), (129, 130, 128, False),
+                                          (300, 100, 384, False), (257, 1000, 192, True), (600, 136, 512, True)])   # K whole
 def test_half_size_tiles_keep_the_bits(ctx, monkeypatch, M, N, K, swiglu):
     """Half-size tiles over the codes (the default at these shapes) add the same
     slices of K as the plan's own tiles over the bf16 expansion
     (VLRF_HIP_PREFILL_DQ=0): the same result to the bit."""
     print(f"[case] half-size tiles M={M} N={N} K={K} swiglu={swiglu}", flush=True)
+    assert gemm_plan(V.DT_Q4_0, M, N, K, swiglu)[2]
     ws = [_weight(ctx, 30, f"H{i}.{N}x{K}", N, K, V.DT_Q4_0)[0] for i in range(1 + swiglu)]
     dx = ctx.to_device(F.normal(30, f"hx{M}x{K}", M * K).reshape(M, K))
     out = []
@@ -328,19 +379,21 @@ def _hip():
 
 
 @pytest.mark.parametrize("dtype", [V.DT_Q8_0, V.DT_Q4_0])
-@pytest.mark.parametrize("M", [160, 64])
-def test_prefill_gemm_under_graph_capture(orc, dtype, M):
+@pytest.mark.parametrize("M,N,K,more", [(160, 512, 1024, 4), (64, 512, 1024, 4), (300, 2051, 2752, 10)])
+def test_prefill_gemm_under_graph_capture(orc, dtype, M, N, K, more):
     """A stream under graph capture: the M > 128 GEMM records no allocation
     (the weight's bf16 expansion is not made, the tiles decode the blocks),
-    the captured graph replays to the eager result (over the expansion) bit
-    for bit, replay after replay with eager work between; a call that would
-    grow the context scratch while capturing is refused with an error
-    instead of being recorded.  M = 64 takes the K-split GEMM and its reduce
-    launch (partial sums in the context scratch after the bf16 rows)."""
+    the captured graph replays to the eager result (at 300 rows over the
+    expansion, at the two others on half-size tiles over the codes) bit
+    for bit, replay after replay with eager work between; a call whose rows
+    alone would grow the context scratch while capturing is refused with an
+    error instead of being recorded.  All three split K (partial sums in the
+    context scratch after the bf16 rows) and launch the reduction."""
     import ctypes as C
     hip = _hip()
     ctx = V.Context(0)                  # its own scratch buffer, empty until the first call
-    N, K = 512, 1024
+    S, _, few, _ = gemm_plan(dtype, M, N, K)
+    assert S > 1 and few == (M != 300)
     print(f"[case] qgemm under capture dtype={dtype} M={M} N={N} K={K}", flush=True)
     w1, dec = _weight(ctx, 31, "cap", N, K, dtype)
     w2, _ = _weight(ctx, 31, "cap", N, K, dtype)              # the same blocks, never expanded
@@ -372,8 +425,8 @@ def test_prefill_gemm_under_graph_capture(orc, dtype, M):
     hip.hipGraphExecDestroy(ge)
     hip.hipGraphDestroy(g)
     # Scratch growth while capturing: refused, the capture ends cleanly.
-    M2 = 4 * M
-    dx2, y3 = ctx.to_device(np.tile(x, (4, 1))), ctx.alloc(M2 * N * 4)
+    M2 = more * M
+    dx2, y3 = ctx.to_device(np.tile(x, (more, 1))), ctx.alloc(M2 * N * 4)
     assert hip.hipStreamBeginCapture(s, 2) == 0
     rc = V.lib().vlrf_hip_qlinear(ctx.h, w1.h, dx2.ptr, y3.ptr, M2, None, C.c_float(0.0), None)
     g = C.c_void_p()

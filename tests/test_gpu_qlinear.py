@@ -216,6 +216,51 @@ def test_small_m_any_k(ctx, dtype, M, N, K, norm, res):
     assert (np.abs(dy.download((M, N)) - ref) <= bound).all()
 
 
+@pytest.mark.parametrize("dtype", [V.DT_Q8_0, V.DT_Q4_0])
+@pytest.mark.parametrize("M,K", [(16, 288), (5, 1056), (3, 4128)])
+def test_small_m_any_k_every_piece_of_x_counts(ctx, dtype, M, K):
+    """x = 1 + small parts that only the second, or only the third, bf16 piece
+    holds, over weights c, -c, c, ..: the first piece (and the second) cancels in
+    every block and the result is the small parts alone.  Of each block's 32
+    products in three pieces, at most 100 additions round, each by eps of a
+    partial sum, which is at most half of the absolute sum; a lost piece is five
+    times that bound off, or more."""
+    N, nb = 70, K // 32
+    print(f"[case] small M pieces M={M} K={K} dtype={dtype}", flush=True)
+    scale = np.frombuffer(np.float16(1 / 64).tobytes(), np.uint8)
+    codes = np.tile(np.array([127, 129], np.uint8), 16) if dtype == V.DT_Q8_0 else np.full(16, 0x1F, np.uint8)
+    blocks = np.tile(np.concatenate([scale, codes]), N * nb).reshape(N, -1)
+    c = (127 if dtype == V.DT_Q8_0 else 7) / 64
+    w = V.QuantWeight(ctx, blocks, dtype, N, K)
+    k = 255 - np.arange(M)[:, None]
+    for base, part in ((1.0, k * 2.0 ** -15), (1.0 + 2.0 ** -8, k * 2.0 ** -23)):
+        x = np.full((M, K), base)
+        x[:, ::2] += part
+        assert (x.astype(np.float32) == x).all()
+        dy = ctx.alloc(M * N * 4)
+        ctx.qlinear(w, ctx.to_device(x.astype(np.float32)), dy, M)
+        ref = c * (K // 2) * part                             # every column of the result alike
+        bound = 100 * 2.0 ** -24 * (c * K * 1.01) / 2
+        assert (ref > 4 * bound).all()
+        assert (np.abs(dy.download((M, N)) - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [V.DT_Q8_0, V.DT_Q4_0])
+def test_small_m_any_k_error_at_long_k(ctx, dtype):
+    """56 slices added with their rounding errors: no further from 64 bits than the
+    vector kernel at this shape (1.6e-7 of the 2-norm; 1.9e-7 without the errors)."""
+    M, N, K = 16, 300, 14272
+    print(f"[case] small M long K dtype={dtype}", flush=True)
+    w, dec = _weight(ctx, 37, f"L{N}x{K}", N, K, dtype)
+    x = F.normal(37, f"x{M}x{K}", M * K).reshape(M, K)
+    dy = ctx.alloc(M * N * 4)
+    ctx.qlinear(w, ctx.to_device(x), dy, M)
+    ref = x.astype(np.float64) @ dec.astype(np.float64).T
+    err = np.linalg.norm(dy.download((M, N)) - ref) / np.linalg.norm(ref)
+    print(f"[error] {err:.3g}", flush=True)
+    assert err <= 1.6e-7
+
+
 @pytest.mark.parametrize("M,N,K,norm,res", [
     (2, 70, 256, True, False), (8, 64, 512, True, True), (9, 63, 2048, True, False), (16, 130, 2304, True, False),
     (7, 65, 2560, False, True), (16, 40, 4352, True, False), (3, 33, 2304, False, False)])
