@@ -72,6 +72,28 @@ def test_gemm_f32_tiles_and_splits(ctx, M, N, K, pad, off, ta, tb):
     assert np.array_equal(got[:, N:], C0[:, N:])                        # between the rows of C
 
 
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (33, 3, 3), (64, 64, 4), (64, 65, 16), (17, 130, 15), (64, 64, 17),
+                                   (2100, 1030, 32), (2100, 1030, 33), (70, 50001, 48), (70, 50001, 49),
+                                   (65, 50000, 80), (65, 50000, 81)])
+def test_gemm_f32_short_k(ctx, M, N, K, ta, tb):
+    """Both sides of the lines between the two kernels: one step of 16, 512 and 1536
+    tiles, K of 32, 48 and 80; alpha, beta and a gap between the rows of C."""
+    print(f"[case] gemm short K M={M} N={N} K={K} ta={ta} tb={tb}", flush=True)
+    A, B = F.normal(71, f"a{M}.{K}", M * K).reshape(M, K), F.normal(71, f"b{K}.{N}", K * N).reshape(K, N)
+    ldc = N + 3
+    C0 = F.normal(71, f"c{M}.{N}", M * ldc).reshape(M, ldc)
+    dA, dB = (ctx.to_device(np.ascontiguousarray(t.T if x else t)) for t, x in ((A, ta), (B, tb)))
+    dC = ctx.to_device(C0)
+    V.check(V.lib().vlrf_hip_gemm_f32(ctx.h, dA.ptr, dB.ptr, dC.ptr, M, N, K, M if ta else K, K if tb else N, ldc,
+                                      1.5, 0.5, int(ta), int(tb)))
+    got = dC.download((M, ldc))
+    ref, mag = _gemm64(A, B)
+    bound = (K + 4) * 2.0 ** -24 * 1.5 * mag + 3 * 2.0 ** -24 * np.abs(0.5 * C0[:, :N].astype(np.float64)) + 1e-30
+    assert (np.abs(got[:, :N] - (1.5 * ref + 0.5 * C0[:, :N])) <= bound).all()
+    assert np.array_equal(got[:, N:], C0[:, N:])
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 40, 200), (70, 130, 1024)])
 def test_gemm_f32_specials(ctx, M, N, K):
     """Infinities, NaN and denormals stay in their row of C and keep their meaning."""

@@ -29,8 +29,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // distinct banks), so lane half h takes k = 8s + 4h + 0..3 in one read (the
 // order of k within a step is the same for both operands, and otherwise free).
 // Products and sums are f32 FMAs as in the CPU loop; infinities and NaN pass
-// through; rows and columns outside the matrices are zeros that no stored
-// element reads.
+// through; rows and columns outside the matrices are copies of the last ones,
+// whose products no stored element takes.
 //
 // Bound by the matrix rate (157 TFLOP/s f32) while the tiles fill the chip,
 // else by the length of a workgroup's own K: the slices of a split K
@@ -175,6 +175,65 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
             *c = prev + alpha * acc[r];
         }
     }
+}
+
+// The same for short K on the vector units: a 256-lane workgroup owns a 64x64 tile
+// of C, each lane a 4x4 block (rows ty + 16i, columns tx + 16j, so LDS reads of a
+// wave are broadcast or conflict-free); K in steps of 16 staged through LDS.
+// Bound by the stores of C and one trip to memory, where a step of 64 is mostly
+// padding and its 68 KiB of LDS leave two workgroups a CU (us, that kernel / this
+// one: 4096 x 4096 x 8 44.8 / 18.3, x 48 45.2 / 39.2, x 64 45.0 / 48.9; 100 x 50000 x 32
+// 21.4 / 15.4; 1 x 4096 x 16 5.2 / 4.1).
+constexpr int kShortT = 64, kShortK = 16;
+
+__global__ __launch_bounds__(256) void gemm_f32_short_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                                                             float* C, int M, int N, int K, int lda, int ldb,
+                                                             int ldc, float alpha, float beta, int transA, int transB) {
+    __shared__ float As[kShortK][kShortT + 1];
+    __shared__ float Bs[kShortK][kShortT + 1];
+    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+    const int m0 = blockIdx.y * kShortT, n0 = blockIdx.x * kShortT;
+    float acc[4][4] = {};
+    for (int k0 = 0; k0 < K; k0 += kShortK) {
+        for (int i = tid; i < kShortT * kShortK; i += 256) {
+            // A tile element (m, k): lanes walk k fastest when A is row-major in k
+            const int r = transA ? i % kShortT : i / kShortK, c = transA ? i / kShortT : i % kShortK;
+            const int m = m0 + r, k = k0 + c;
+            float a = 0.f;
+            if (m < M && k < K) a = transA ? A[(size_t)k * lda + m] : A[(size_t)m * lda + k];
+            As[c][r] = a;
+            const int rb = transB ? i / kShortK : i % kShortT, cb = transB ? i % kShortK : i / kShortT;   // (n, k)
+            const int n = n0 + rb, kb = k0 + cb;
+            float b = 0.f;
+            if (n < N && kb < K) b = transB ? B[(size_t)n * ldb + kb] : B[(size_t)kb * ldb + n];
+            Bs[cb][rb] = b;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int kk = 0; kk < kShortK; ++kk) {
+            float a[4], b[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty + 16 * i];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx + 16 * j];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int m = m0 + ty + 16 * i, n = n0 + tx + 16 * j;
+            if (m < M && n < N) {
+                float* c = C + (size_t)m * ldc + n;
+                const float prev = beta == 0.f ? 0.f : (beta == 1.f ? *c : *c * beta);
+                *c = prev + alpha * acc[i][j];
+            }
+        }
 }
 
 // C = beta*C + alpha * (the S slices' partial sums, in slice order).
@@ -367,6 +426,20 @@ GemmF32Plan gemm_f32_plan(int M, int N, int K) {
     return p;
 }
 
+// Where K is short (it then stays whole) and the vector-unit kernel faster: one step
+// of its 16, but for aligned operands of up to 256 tiles, and more of them as the
+// tiles take more rounds of the other's two workgroups a CU.  us, steps of 64 / of
+// 16: 1024 x 1024 x 16 5.5 / 6.2 (A transposed, x 4 6.6 / 6.0); 1024 x 2048 x 16 7.7 / 6.7,
+// x 32 7.7 / 9.1; 1536 x 1536 x 32 10.5 / 9.2, x 48 10.5 / 11.7; 3072 x 3072 x 48 26.6 /
+// 24.4, x 64 26.9 / 30.0, x 72 39.3 / 37.4 (B transposed 34.6 / 36.8); 16 x 200000 x 96
+// 57.9 / 49.9.
+bool gemm_f32_short(int M, int N, int K, bool transA, bool transB, bool vec) {
+    const long tiles = (long)((M + kShortT - 1) / kShortT) * ((N + kShortT - 1) / kShortT);
+    if (K <= 16) return !(vec && !transA && K >= 4 && M >= 64 && N >= 64 && tiles <= 256);
+    if (K <= 32) return tiles > 512;
+    return tiles >= 1536 && (K <= 48 || (K > 64 && K <= (M <= 32 ? 96 : 80) && !transB));
+}
+
 }  // namespace
 
 size_t gemm_f32_part_bytes(int M, int N, int K) {
@@ -388,6 +461,13 @@ int launch_gemm_f32(hipStream_t s, const float* A, const float* B, float* C, int
     float* P = p.S > 1 ? part : nullptr;
     const bool va = ((uintptr_t)A & 15) == 0 && lda % 4 == 0 && lda < (1 << 22) && (transA ? M : K) % 4 == 0;
     const bool vb = ((uintptr_t)B & 15) == 0 && ldb % 4 == 0 && ldb < (1 << 22) && (transB ? K : N) % 4 == 0;
+    if (gemm_f32_short(M, N, K, transA, transB, va && vb)) {
+        const dim3 grid((N + kShortT - 1) / kShortT, (M + kShortT - 1) / kShortT);
+        hipLaunchKernelGGL(gemm_f32_short_kernel, grid, dim3(256), 0, s, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta,
+                           (int)transA, (int)transB);
+        VH_LAUNCHED();
+        return VLRF_HIP_OK;
+    }
     const int bm = p.wide ? 32 : 64, bn = p.wide ? 128 : 64;
     const dim3 grid((N + bn - 1) / bn, (M + bm - 1) / bm, p.S);
 #define VH_GF(BM, BN, TA, TB, VV)                                                                               \
