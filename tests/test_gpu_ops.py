@@ -245,7 +245,8 @@ def test_gelu_and_add_groups_of_four(ctx, orc, n, off):
     assert (np.delete(s, np.s_[off:off + n]) == 9.0).all() and (np.delete(g, np.s_[off:off + n]) == 9.0).all()
 
 
-@pytest.mark.parametrize("rows,D,off", [(5, 4, 0), (3, 1020, 0), (2, 1028, 0), (2, 4096, 0), (2, 4100, 0), (3, 768, 1)])
+@pytest.mark.parametrize("rows,D,off", [(5, 4, 0), (3, 1020, 0), (2, 1028, 0), (2, 4096, 0), (2, 4100, 0), (3, 768, 1),
+                                        (3, 1024, 0), (2, 2048, 0), (2, 2052, 0), (3000, 64, 0)])
 def test_layer_norm_in_registers(ctx, rows, D, off):
     """Row lengths at the edges of the register form, and addresses that forbid it,
     against 64 bits: every step is an f32 sum of D terms."""

@@ -291,31 +291,33 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const float* __restrict
     for (int j = threadIdx.x; j < D; j += 256) o[j] = (r[j] - mean) * inv * w[j] + b[j];
 }
 
-// Rows of up to 4096 columns held in registers, four float4 a thread: read once, and
-// no load behind a reduction (a call among others, 1000 x 1600: 5.3 -> 4.4 us; 300 x 768
-// 3.7 -> 3.5, near what a launch costs).
+// Rows of up to 4096 columns held in registers, NV float4 a thread (as many as the
+// row has thousands of columns: with all four for every row, 20000 x 64 took 28.8 us):
+// read once, and no load behind a reduction.  Against the kernel above, us: 1000 x
+// 1600 5.1 -> 3.75, 4000 x 768 7.4 -> 5.5, 20000 x 1024 42.6 -> 24.4, 20000 x 64 10.8 -> 10.8.
+template <int NV>
 __global__ __launch_bounds__(256) void layer_norm_regs_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                               const float* __restrict__ b, float* out, int D,
                                                               float eps) {
     __shared__ float red[4];
     const float4* r = reinterpret_cast<const float4*>(x + (size_t)blockIdx.x * D);
     const int n4 = D / 4;
-    float4 v[4], wv[4], bv[4];
+    float4 v[NV], wv[NV], bv[NV];
     float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NV; ++i) {
         const int j = min((int)threadIdx.x + 256 * i, n4 - 1);
         v[i] = r[j];
         wv[i] = reinterpret_cast<const float4*>(w)[j];
         bv[i] = reinterpret_cast<const float4*>(b)[j];
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NV; ++i)
         if ((int)threadIdx.x + 256 * i < n4) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
     const float mean = block_sum(s, red) / (float)D;
     float q = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NV; ++i) {
         v[i] = make_float4(v[i].x - mean, v[i].y - mean, v[i].z - mean, v[i].w - mean);
         if ((int)threadIdx.x + 256 * i < n4)
             q += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
@@ -324,7 +326,7 @@ __global__ __launch_bounds__(256) void layer_norm_regs_kernel(const float* __res
     const float inv = 1.f / sqrtf(var);
     float4* o = reinterpret_cast<float4*>(out + (size_t)blockIdx.x * D);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NV; ++i) {
         const int j = threadIdx.x + 256 * i;
         if (j < n4)
             o[j] = make_float4(v[i].x * inv * wv[i].x + bv[i].x, v[i].y * inv * wv[i].y + bv[i].y,
@@ -501,8 +503,13 @@ int launch_gemm_f32(hipStream_t s, const float* A, const float* B, float* C, int
 int launch_layer_norm(hipStream_t s, const float* x, const float* w, const float* b, float* out, int rows, int D,
                       float eps) {
     VH_ARG(x && w && b && out && rows >= 1 && D >= 1, "layer_norm: bad arguments");
-    if (D % 4 == 0 && D <= 4096 && aligned16(x, w, b, out))
-        hipLaunchKernelGGL(layer_norm_regs_kernel, dim3(rows), dim3(256), 0, s, x, w, b, out, D, eps);
+    const bool regs = D % 4 == 0 && D <= 4096 && aligned16(x, w, b, out);
+    if (regs && D <= 1024)
+        hipLaunchKernelGGL(layer_norm_regs_kernel<1>, dim3(rows), dim3(256), 0, s, x, w, b, out, D, eps);
+    else if (regs && D <= 2048)
+        hipLaunchKernelGGL(layer_norm_regs_kernel<2>, dim3(rows), dim3(256), 0, s, x, w, b, out, D, eps);
+    else if (regs)
+        hipLaunchKernelGGL(layer_norm_regs_kernel<4>, dim3(rows), dim3(256), 0, s, x, w, b, out, D, eps);
     else
         hipLaunchKernelGGL(layer_norm_kernel, dim3(rows), dim3(256), 0, s, x, w, b, out, D, eps);
     VH_LAUNCHED();
