@@ -216,6 +216,22 @@ def test_small_m_any_k(ctx, dtype, M, N, K, norm, res):
     assert (np.abs(dy.download((M, N)) - ref) <= bound).all()
 
 
+@pytest.mark.parametrize("M,N,K,norm", [(4, 60, 512 - 32, False), (4, 60, 544, False), (3, 60, 992, False), (3, 60, 1056, False),
+                                        (2, 8193, 1056, False), (2, 8192, 1056, False), (3, 16385, 608, False),
+                                        (2, 60, 992, True), (3, 60, 704, True)])
+def test_small_m_any_k_lines_between_the_kernels(ctx, M, N, K, norm):
+    """Either side of where such calls go over from the vector kernel: the same
+    bound on both (it is theirs, not a kernel's)."""
+    print(f"[case] small M lines M={M} N={N} K={K} norm={norm}", flush=True)
+    w, dec = _weight(ctx, 38, f"W{N}x{K}", N, K, V.DT_Q4_0)
+    x = F.normal(38, f"x{M}x{K}", M * K).reshape(M, K)
+    nw = 1 + F.normal(38, f"n{K}", K, 0.1) if norm else None
+    dy = ctx.alloc(M * N * 4)
+    ctx.qlinear(w, ctx.to_device(x), dy, M, norm_w=ctx.to_device(nw) if norm else None)
+    ref, bound = _small_bound(x, dec, nw)
+    assert (np.abs(dy.download((M, N)) - ref) <= bound).all()
+
+
 @pytest.mark.parametrize("dtype", [V.DT_Q8_0, V.DT_Q4_0])
 @pytest.mark.parametrize("M,K", [(16, 288), (5, 1056), (3, 4128)])
 def test_small_m_any_k_every_piece_of_x_counts(ctx, dtype, M, K):

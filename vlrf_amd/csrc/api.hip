@@ -647,18 +647,37 @@ static int gemm_scratch(Ctx* ctx, size_t a_bytes, size_t p_bytes, float** a, flo
     return VLRF_HIP_OK;
 }
 
+// The M K columns of work from which K in other than whole slices runs faster on the
+// small-M kernel than on the vector kernel.  That takes 4 or 16 rows at a time (so M
+// of 5 and more gains most) and K in passes of 1024, fills the CUs best with 8193 ..
+// 16384 rows of weights (SwiGLU from 6145), and reads x twice with a fused norm; the
+// small-M kernel decodes Q4_0 slower than Q8_0.  us, vector / small-M kernel:
+//   M = 5      1000 x 384 Q8_0 9.1 / 5.5, 14000 x 832 Q8_0 49 / 11.3; M = 16 14000 x 14272 1640 / 84
+//   M = 4      300 x 480 Q8_0 5.0 / 5.5, x 544 5.3 / 5.0; 14000 x 832 Q8_0 8.8 / 9.7
+//   M = 3      300 x 800 Q8_0 6.2 / 5.8, Q4_0 5.4 / 5.8; 5000 x 1056 Q4_0 8.0 / 6.8;
+//              32000 x 608 Q8_0 13.4 / 11.0; 14000 x 1344 Q8_0 11.4 / 12.2
+//   M = 2      5000 x 960 Q4_0 5.3 / 6.7, x 1056 7.4 / 6.9; 32000 x 960 Q8_0 18.0 / 15.4;
+//              14000 x 1344 Q8_0 10.9 / 12.7, x 2112 15.7 / 13.3
+//   SwiGLU     M = 2 1000 x 1440 Q8_0 9.7 / 7.0, 14000 x 1440 Q4_0 16.1 / 18.8; M = 16 5361 x 8000 Q4_0 414 / 35
+//   norm       M = 2 5000 x 960 Q4_0 7.0 / 7.6, Q8_0 7.9 / 7.6; M = 4 14000 x 480 9.5 / 7.6
+static long small_from(int M, int N, bool two, bool norm, bool q4) {
+    const bool full = N > (two ? 6144 : 8192) && N <= 16384, many = N > 16384;
+    long from = 1800;
+    if (norm && M <= 4) from = q4 && N <= 8192 ? 2049 : 1800;
+    else if (M == 4) from = full ? (q4 || two ? 1800 : 4097) : many ? 1800 : 2049;
+    else if (M == 3) from = many ? 1800 : q4 || full ? 3073 : 2400;
+    else if (M == 2) from = full ? (q4 ? 4100 : two ? 2800 : 3700) : many && !q4 ? 1800 : 2049;
+    return two ? std::max(from, 2800L) : from;
+}
+
 // Scratch of the small-M kernel (2 <= M <= 16); null: the call runs on the vector
 // kernel.  K in whole slices always takes it (an error where the scratch cannot
-// be had); any other K from M K columns of work on, unless the scratch is out
-// of reach (under capture, beyond the tile counters or 2 GiB of partials).  The
-// line, us on the vector kernel / this one at Q8_0: M = 2, 300 x 448 4.3 / 5.2,
-// 14000 x 832 9.2 / 10.4, 14000 x 1344 13.8 / 12.5; M = 3, 300 x 832 6.2 / 5.1; M = 7,
-// 402 x 320 10.2 / 5.4; M = 16, 14000 x 14272 1640 / 84; SwiGLU, M = 2, 14000 x 1344
-// 17.9 / 18.6, 300 x 2112 14.2 / 8.1; M = 16, 5361 x 8000 414 / 35.
-static int small_scratch(Ctx* ctx, const DevWeight& w, int M, bool two, float** out) {
+// be had); any other K from small_from on, unless the scratch is out of reach
+// (under capture, beyond the tile counters or 2 GiB of partials).
+static int small_scratch(Ctx* ctx, const DevWeight& w, int M, bool two, bool norm, float** out) {
     const size_t need = qlinear_small_scratch(w.N, w.K, two);
     if (qlinear_small_whole(w)) return ctx->scratch(need, out);
-    const bool pays = (long)M * w.K >= (two ? 2800 : 1800);
+    const bool pays = (long)M * w.K >= small_from(M, w.N, two, norm, w.dtype == VLRF_HIP_DT_Q4_0);
     *out = pays && qlinear_small_tiles(w.N) <= kSmallMaxTiles && need < 0x7fffffffu ? ctx->try_scratch(need) : nullptr;
     return VLRF_HIP_OK;
 }
@@ -675,7 +694,7 @@ int vlrf_hip_qlinear(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t w, const float* x, fl
     VH_ARG(x != y, "qlinear: x must not alias y");
     float* scratch_m = nullptr;
     if (M >= 2 && M <= 16 && qlinear_small_supported(w->w)) {
-        int rc = small_scratch(ctx, w->w, M, false, &scratch_m);
+        int rc = small_scratch(ctx, w->w, M, false, norm_w != nullptr, &scratch_m);
         if (rc) return rc;
     }
     if (scratch_m)
@@ -701,7 +720,7 @@ int vlrf_hip_qlinear_swiglu(vlrf_hip_ctx_t ctx, vlrf_hip_weight_t wg, vlrf_hip_w
     VH_ARG(x != h, "swiglu: x must not alias h");
     float* scratch_m = nullptr;
     if (M >= 2 && M <= 16 && qlinear_small_supported(wg->w)) {
-        int rc = small_scratch(ctx, wg->w, M, true, &scratch_m);
+        int rc = small_scratch(ctx, wg->w, M, true, norm_w != nullptr, &scratch_m);
         if (rc) return rc;
     }
     if (scratch_m)
