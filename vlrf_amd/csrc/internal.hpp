@@ -187,8 +187,8 @@ int launch_rows_to_bf16(hipStream_t s, const float* x, const float* w, uint16_t*
                         float eps);
 // y[M,N] = a[M,K] . W^T (+ residual), a in bf16, W Q8_0/Q4_0 with K % 64 == 0.
 // `part`: device memory of qgemm_part_bytes(w, M, false) bytes for the K-split
-// partial sums of 17 <= M <= 128 (without it such a call takes the unsplit
-// register-staged kernel).
+// partial sums of M > 16 (without it K stays whole: up to 128 rows on the
+// register-staged kernel, above on the unsplit plans).
 int launch_qgemm(hipStream_t s, const DevWeight& w, const uint16_t* a, int M, const float* residual,
                  float* y, float* part = nullptr);
 // h[M,N] = silu(a.Wg^T) * (a.Wu^T), stored as bf16 (h_bf16) or f32

@@ -873,9 +873,10 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(
 // Bound by the matrix rate and, beside it, the softmax's vector work (about 300
 // instructions to the 64 matrix instructions of a tile at d 64, two waves a
 // SIMD).  Measured against one thread a query on the vector units (32 heads, d
-// 64, causal): 777 x 777 keys 766 -> 41 us, 1024 x 1024 997 -> 54 (79
-// TFLOP/s); d 128, 1024 x 2048 keys 7205 -> 286; 12 heads, 41 x 568 474 -> 15.
-// Plain 64-bit addresses ran 64.6, these loads 41; eight waves a block 44.6.
+// 64, causal): 777 x 777 keys 767 -> 37.5 us (66 TFLOP/s over the causal half);
+// all of 1024 x 1024 78; d 128, 700 x 700 75; 12 heads, 500 x 900 22.7; 33 x 33 5.7.
+// In an earlier form, plain 64-bit addresses ran 64.6 us at 777 x 777 where these
+// loads ran 41 and eight waves a block 44.6.
 //
 // Weights are exp2(s * sl2 - m * sl2) with one rounding at the difference's
 // size, the scores' sums run in four chains and the result is one division: the
@@ -1678,12 +1679,12 @@ int launch_attn_decode(hipStream_t s, const float* q, const void* kc, const void
     if (!fuse && !chunked) {
         // Workgroups of four waves, a round of 8 KiB of K per wave (rr8 rows), as
         // many rounds as leave about one workgroup per CU (it holds 300 registers a
-        // lane: 512 ran 25.9 against 22.2 us at 15001 keys, 8 KV heads, d 128, f16).
+        // lane: 512 ran 25.9 us at 15001 keys, 8 KV heads, d 128, f16, 256 22.2).
         // Fewer workgroups than CUs: rounds of a quarter of that, so four times as
         // many (32/8 heads, d 128, Q8_0 4096: 13.3 -> 12.2 us; 8/2 heads, 582: 11.6 ->
         // 9.3), unless one chunk holds all the keys and needs no merge.
         // Before: 64-key workgroups and a serial merge of their partials, 56.3 us
-        // at 15001 keys f16 (100.2 f32, 44.5 Q8_0), now 22.3 (28.5, 20.8).
+        // at 15001 keys f16 (100.2 f32, 44.5 Q8_0), now 21.2 (28.5, 20.8).
         VH_ARG(!ctx_dev, "attn_decode: a device position needs the fused form");
         const float sl2 = (float)(std::fabs((double)scale) * 1.4426950408889634), qsign = scale < 0.f ? -1.f : 1.f;
         const int hg = rep < 4 ? rep : 4, groups = n_heads / hg;

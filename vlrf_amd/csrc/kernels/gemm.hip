@@ -1467,7 +1467,11 @@ KSplit split_k(long tiles, int K, int cus, int least = 8) {
 // and both forms above 128 rows agree to the bit whichever tiles each takes.  us, the
 // plan's tiles / these / these in slices of their own: 1.1B QKV at M = 233 20.3 /
 // 18.9 / 17.2, O 19.1 / 16.0 / 16.0; 1024 x 1024, M = 256, 15.8 / 13.0 / 12.2;
-// 397 x 4096, M = 108, 17.1 / 15.0 / 16.5; 4343 x 1280, M = 166, 19.9 / 18.8 / 14.2.
+// 397 x 4096, M = 108, 17.1 / 15.0 / 16.5.  Beyond 1.25 rounds of the CUs in such
+// slices (SwiGLU, whose own tiles are eight times these, 2.5) the plan's tiles
+// stay: over 60 drawn shapes above 128 rows these take 0.79 .. 0.91 of their time up
+// to one round, 0.92 .. 1.07 from there on, SwiGLU 0.58 .. 0.85 to two rounds,
+// 0.95 .. 1.01 to three, then up to 1.14.
 // Any other K takes at most 24 slices of at least 4 steps, but not two slices of
 // up to 16 steps, which do not pay for their reduction: 1236 x 1344, M = 38, 15.5 ->
 // 11.0; 345 x 1216, M = 324, 17.0 -> 12.1; 2270 x 1216, M = 434, 22.9 -> 15.7; SwiGLU
@@ -1482,7 +1486,9 @@ KSplit few_split(const DevWeight& w, int M, bool swiglu, const KSplit& own, long
     const long few = (long)((M + bm - 1) / bm) * ((w.N + bn - 1) / bn);
     if (2 * few > 5L * cus) return own;
     KSplit ks = own;
-    if (own.S == 1 || w.K % (128 * own.S)) {
+    if (own.S > 1 && w.K % (128 * own.S) == 0) {
+        if (4 * few * own.S > (swiglu ? 10L : 5L) * cus) return own;
+    } else {
         ks = split_k(few, w.K, cus < 24 * few ? cus : (int)(24 * few), 4);
         if (ks.S == 2 && w.K <= 16 * 64) ks = {1, w.K};
     }
@@ -1548,6 +1554,9 @@ void launch_dq_split(hipStream_t s, const uint16_t* a, const DevWeight& w0, cons
 // at least 8 K steps (split_k) -- with
 // the partial buffer and splitk_reduce_kernel of the 17..128-row path, so
 // the two forms still multiply and add the same numbers in the same order.
+// (Half-size tiles run over the codes in both settings; where
+// VLRF_HIP_PREFILL_DQ=0 keeps them out, slices that few_split does not keep
+// from the plan are others there.)
 // (8B layer, same box: against aiming at 3/4 of a round from below half a
 // round, T = 1024 0.677 -> 0.600 ms, its O and down now split in two; T =
 // 256 .. 768 within noise.  Aiming at a full round: T = 256 0.291 ms.)
@@ -2148,7 +2157,7 @@ int launch_qgemm(hipStream_t s, const DevWeight& w, const uint16_t* a, int M, co
     if (rc) return rc;
     VH_ARG(a && y, "qgemm: null operand");
     if (M > 128) {
-        weight_expand_bf16(s, w);
+        weight_expand_bf16(s, w);   // also where half-size tiles read the codes: other row counts read it
         const KSplit ks = part || !qgemm_part_bytes(w, M, false) ? gemm_split(w, M, false) : KSplit{1, w.K};
         if (ks.few) {
             if (residual) launch_dq_split<1>(s, a, w, nullptr, M, ks, residual, y, part);
